@@ -8,8 +8,7 @@ requires it), the same C-ABI call also runs the hand-written adjoint, so ``J.bac
 dJ/dgamma and dJ/du_peak without further GPU work; otherwise (``torch.no_grad()``, line searches,
 finite differences) only the steps and the objective run (``cfd_lbm_objective_run``), the same J
 bit for bit at the cost of the forward steps alone.  A ``gamma`` on the GPU stays there: the field
-is read from device memory and, with binomial checkpointing, dJ/dgamma is written into a device
-tensor; no host round trip.  PyTorch is only the caller's interface here: the forward steps, the
+is read from device memory and dJ/dgamma is written into a device tensor; no host round trip.  PyTorch is only the caller's interface here: the forward steps, the
 transposed steps and the checkpointing all run in ``libcfd_lbm_hip.so``.
 
 The reference has no differentiable solver; the gradients are checked against central finite
@@ -97,18 +96,28 @@ class LbmAdjointProblem:
     def run(self, gamma, u_peak: float):
         """J, dJ/dgamma (float64, shape of gamma; a device tensor when gamma is one and the plan is
         binomial, else a numpy array) and dJ/du_peak from one forward + adjoint run."""
+        J, grad, du = self._run(gamma, u_peak)
+        if self.checkpoint_every > 0 and isinstance(grad, torch.Tensor):
+            grad = grad.cpu().numpy()
+        return J, grad, du
+
+    def _run(self, gamma, u_peak: float):
+        """``run`` with dJ/dgamma on the device whenever gamma is."""
         s = self._prepare(gamma, u_peak)
         x_out = self._x_out()
-        if self.checkpoint_every > 0:
-            if self.objective != "pressure_drop":
-                raise ValueError("two-level checkpointing runs the pressure-drop objective; use checkpoint_every=0")
-            J, grad, du = s.adjoint_run(self.steps, self.window, self.checkpoint_every, self.x_in, x_out)
-        elif isinstance(gamma, torch.Tensor) and gamma.is_cuda:
+        if self.checkpoint_every > 0 and self.objective != "pressure_drop":
+            raise ValueError("two-level checkpointing runs the pressure-drop objective; use checkpoint_every=0")
+        if isinstance(gamma, torch.Tensor) and gamma.is_cuda:
             grad = torch.empty(s.cells, dtype=torch.float64, device=gamma.device)
-            torch.cuda.current_stream(grad.device).synchronize()
-            J, du, _ = s.adjoint_run_binomial_device(self.steps, self.window, grad.data_ptr(), self.snapshots,
-                                                     self.objective, self.x_in, x_out)
-            return J, grad.reshape(gamma.shape), du
+            torch.cuda.current_stream(grad.device).synchronize()  # its memory may still be in use there
+            if self.checkpoint_every > 0:
+                J, du = s.adjoint_run_device(self.steps, self.window, self.checkpoint_every, grad.data_ptr(),
+                                             self.x_in, x_out)
+            else:
+                J, du, _ = s.adjoint_run_binomial_device(self.steps, self.window, grad.data_ptr(), self.snapshots,
+                                                         self.objective, self.x_in, x_out)
+        elif self.checkpoint_every > 0:
+            J, grad, du = s.adjoint_run(self.steps, self.window, self.checkpoint_every, self.x_in, x_out)
         else:
             J, grad, du, _ = s.adjoint_run_binomial(self.steps, self.window, self.snapshots, self.objective,
                                                     self.x_in, x_out)
@@ -130,7 +139,7 @@ class LbmObjective(torch.autograd.Function):
             J = problem.evaluate(gamma, u)
             ctx.save_for_backward(torch.zeros_like(gamma), torch.zeros_like(u_peak))
             return torch.tensor(J, dtype=torch.float64, device=gamma.device)
-        J, grad, du = problem.run(gamma, u)
+        J, grad, du = problem._run(gamma, u)
         if not isinstance(grad, torch.Tensor):
             grad = torch.from_numpy(grad)
         ctx.save_for_backward(grad.to(gamma.device, gamma.dtype),

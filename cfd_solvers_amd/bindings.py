@@ -75,6 +75,8 @@ _SIGNATURES = {
     "cfd_lbm_objective_run": [C.c_void_p, C.c_int, C.c_uint64, C.c_uint64, C.c_int, C.c_int, C.POINTER(C.c_double)],
     "cfd_lbm_adjoint_run": [C.c_void_p, C.c_uint64, C.c_uint64, C.c_uint64, C.c_int, C.c_int,
                             C.POINTER(C.c_double), C.c_void_p, C.POINTER(C.c_double)],
+    "cfd_lbm_adjoint_run_device": [C.c_void_p, C.c_uint64, C.c_uint64, C.c_uint64, C.c_int, C.c_int,
+                                   C.POINTER(C.c_double), C.c_void_p, C.POINTER(C.c_double)],
     "cfd_lbm_adjoint_timing": [C.c_void_p, C.POINTER(C.c_float), C.POINTER(C.c_float)],
     "cfd_lbm_set_drag_body": [C.c_void_p, C.c_void_p, C.c_int],
     "cfd_lbm_set_smagorinsky": [C.c_void_p, C.c_int],
@@ -426,6 +428,15 @@ class EsotericPullHipSolver:
         self.lib.call("cfd_lbm_adjoint_run", self._h, steps, window, checkpoint_every, x_in, x_out, C.byref(J),
                       grad.ctypes.data if grad is not None else None, C.byref(du))
         return J.value, (grad.reshape(self.shape) if grad is not None else None), du.value
+
+    def adjoint_run_device(self, steps, window, checkpoint_every, grad_device, x_in=1, x_out=None):
+        """adjoint_run with dJ/dgamma written to the device address grad_device (cells doubles): J and
+        dJ/du_peak."""
+        J, du = C.c_double(), C.c_double()
+        x_out = self.shape[-1] - 2 if x_out is None else x_out
+        self.lib.call("cfd_lbm_adjoint_run_device", self._h, steps, window, checkpoint_every, x_in, x_out, C.byref(J),
+                      C.c_void_p(int(grad_device)), C.byref(du))
+        return J.value, du.value
 
     def set_smagorinsky(self, enabled=True):
         """The reference's smagorinsky_les switch (esoteric_pull.hpp:72-97, 422-425)."""

@@ -7,6 +7,7 @@
 // src/python/c_api.cpp:8-15: 0 ok, 1 std::exception, 2 unknown, message in a caller buffer.
 #include "../../include/cfd_lbm/c_api.h"
 #include "checkpoint_schedule.hpp"
+#include "device_memory.hpp"
 #include "lbm_adjoint.hpp"
 #include "lbm_kernels.hpp"
 #include "solver_view.hpp"
@@ -63,7 +64,7 @@ template <class T> struct DeviceBuffer {
     void allocate(size_t n_bytes) {
         reset();
         void* p = nullptr;
-        hip_check(hipMalloc(&p, n_bytes), "hipMalloc");
+        hip_check(cfd_hip::device_malloc(&p, n_bytes), "hipMalloc");
         ptr = static_cast<T*>(p);
         bytes = n_bytes;
     }
@@ -86,14 +87,18 @@ __global__ void __launch_bounds__(256) zero_words_kernel(uint32_t* p, uint64_t w
 }  // namespace
 
 namespace {
-// Porosity from device memory: gamma (cells floats) into the solver's plane of `real_bytes`-wide
-// reals; `bad` counts the values outside [0, 1] (NaN included).
+// Porosity from device memory (cells floats): `bad` counts the values outside [0, 1] (NaN included).
+__global__ void __launch_bounds__(256) check_porosity(const float* __restrict__ src, uint64_t cells, uint32_t* bad) {
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const bool wrong = i < cells && !(src[i] >= 0.0F && src[i] <= 1.0F);
+    if (wrong) atomicAdd(bad, 1U);
+}
+// The checked field into the solver's plane of `real_bytes`-wide reals.
 __global__ void __launch_bounds__(256) porosity_from_device(const float* __restrict__ src, void* __restrict__ dst,
-                                                            uint32_t real_bytes, uint64_t cells, uint32_t* bad) {
+                                                            uint32_t real_bytes, uint64_t cells) {
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= cells) return;
     const float g = src[i];
-    if (!(g >= 0.0F && g <= 1.0F)) atomicAdd(bad, 1U);
     if (real_bytes == 4) static_cast<float*>(dst)[i] = g;
     else static_cast<double*>(dst)[i] = static_cast<double>(g);
 }
@@ -251,6 +256,7 @@ struct cfd_lbm_solver {
         try {
             f.allocate(pop_elems * elem);
             initialize_uniform(1.0F, 0.0F, 0.0F, 0.0F);
+            cfd_hip::WorkspacePool::instance().enter();
         } catch (...) {
             (void)hipStreamDestroy(stream);
             throw;
@@ -263,6 +269,7 @@ struct cfd_lbm_solver {
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
         }
+        cfd_hip::WorkspacePool::instance().leave();
     }
 
     void use_device() const { hip_check(hipSetDevice(device), "hipSetDevice"); }
@@ -896,9 +903,10 @@ struct cfd_lbm_solver {
         // starts as aligned as the allocation (hipMalloc: at least 256 B) whatever nx is; the
         // unpadded state size is odd for odd nx.
         const size_t pitch = (state_bytes + 4095) & ~static_cast<size_t>(4095);
-        const size_t fixed = pop_elems * real + 2 * cells * 8 + 64;
+        const size_t fixed = pop_elems * real + 2 * cells * 8 + 8 * 4096;  // with the padding and sums below
         size_t free_b = 0, total_b = 0;
         hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        free_b += cfd_hip::WorkspacePool::instance().idle_bytes();  // given back on demand
         size_t buffers = 0;  // state buffers besides f
         if (every > 0) {
             buffers = static_cast<size_t>((steps + every - 1) / every + std::min<uint64_t>(every, steps) - 1);
@@ -916,26 +924,30 @@ struct cfd_lbm_solver {
             throw std::invalid_argument("checkpoints do not fit in device memory (" + std::to_string(need >> 20) +
                                         " MiB needed, " + std::to_string(free_b >> 20) +
                                         " MiB free): raise the checkpoint interval or lower the snapshot count");
-        // One allocation for all checkpoint states, one buffer every `pitch` bytes.
-        DeviceBuffer<unsigned char> pool_mem;
-        pool_mem.allocate(buffers * pitch);
+        // One block, kept for the next call: the checkpoint states, one every `pitch` bytes, then
+        // lambda, the two gradient accumulators and the sums, each on its own 4 KiB boundary.
+        const auto padded = [](size_t b) { return (b + 4095) & ~static_cast<size_t>(4095); };
+        const size_t lam_at = buffers * pitch, gp_at = lam_at + padded(pop_elems * real);
+        const size_t gg_at = gp_at + padded(cells * sizeof(double));
+        const size_t acc_at = gg_at + (grad_on_device ? 0 : padded(cells * sizeof(double)));
+        const size_t bytes = acc_at + (cfd_hip::kSumBlocks + 2) * sizeof(double);
+        cfd_hip::Workspace block(bytes);
+        unsigned char* const base = block.get();
         std::vector<void*> pool(buffers);
         for (size_t k = 0; k < buffers; ++k) {
-            pool[k] = pool_mem.ptr + k * pitch;
+            pool[k] = base + k * pitch;
             if (reinterpret_cast<uintptr_t>(pool[k]) % 256 != 0)
                 throw std::runtime_error("checkpoint buffer is not 256-byte aligned");
         }
-        DeviceBuffer<unsigned char> lam, gg, gp, acc;
-        lam.allocate(pop_elems * real);
-        if (!grad_on_device) gg.allocate(cells * sizeof(double));
-        gp.allocate(cells * sizeof(double));
-        acc.allocate(sizeof(double));
-        args.grad_gamma = grad_on_device ? grad_gamma_out : reinterpret_cast<double*>(gg.ptr);
-        args.grad_peak = reinterpret_cast<double*>(gp.ptr);
+        void* const lam = base + lam_at;
+        double* const acc = reinterpret_cast<double*>(base + acc_at);
+        double* const peak_sums = acc + 1;
+        args.grad_gamma = grad_on_device ? grad_gamma_out : reinterpret_cast<double*>(base + gg_at);
+        args.grad_peak = reinterpret_cast<double*>(base + gp_at);
         const LaunchState st = state();
         adj->zero(st, args.grad_gamma, cells);
         adj->zero(st, args.grad_peak, cells);
-        adj->zero(st, reinterpret_cast<double*>(acc.ptr), 1);
+        adj->zero(st, acc, 1);
         const bool b = bounded();
         const uint64_t t0 = t;
         const auto par = [t0](uint64_t k) { return ((t0 + k) & 1U) != 0U; };
@@ -984,14 +996,14 @@ struct cfd_lbm_solver {
             ops->step(st, par(k), b, false, cur, dst);
             cur = dst;
             ++forward_steps;
-            if (k + 1 >= steps - window + 1) adj->objective(st, par(k + 1), b, cur, args, 1.0, reinterpret_cast<double*>(acc.ptr));
+            if (k + 1 >= steps - window + 1) adj->objective(st, par(k + 1), b, cur, args, 1.0, acc);
             if (progress > 0 && (k + 1) % progress == 0) report("forward sweep", k + 1, steps);
         }
         t = t0 + steps;
         hip_check(hipEventRecord(e1, stream), "hipEventRecord");
         const auto transposed = [&](uint64_t tt, const void* state) {
             args.add_objective = tt + window >= steps + 1 ? 1 : 0;
-            adj->step(st, par(tt), b, state, lam.ptr, args);
+            adj->step(st, par(tt), b, state, lam, args);
             ++transposed_done;
             if (progress > 0 && transposed_done % progress == 0) report("reverse", transposed_done, steps);
         };
@@ -1002,7 +1014,7 @@ struct cfd_lbm_solver {
             forward_steps += m - a0;
         };
         args.add_objective = 0;
-        adj->seed(st, par(steps), b, lam.ptr, args);
+        adj->seed(st, par(steps), b, lam, args);
         if (every > 0) {
             const uint64_t segments = shots.size();
             for (uint64_t c = segments; c-- > 0;) {
@@ -1038,15 +1050,14 @@ struct cfd_lbm_solver {
         }
         hip_check(hipEventRecord(e2, stream), "hipEventRecord");
         // dJ/du_peak: the inlet cells' contributions summed on the device (fixed order).
-        DeviceBuffer<unsigned char> peak_sums;
-        peak_sums.allocate((cfd_hip::kSumBlocks + 1) * sizeof(double));
-        double* peak_out = reinterpret_cast<double*>(peak_sums.ptr) + cfd_hip::kSumBlocks;
-        adj->sum(st, args.grad_peak, cells, reinterpret_cast<double*>(peak_sums.ptr), peak_out);
+        double* const peak_out = peak_sums + cfd_hip::kSumBlocks;
+        adj->sum(st, args.grad_peak, cells, peak_sums, peak_out);
         double J = 0.0, du = 0.0;
-        d2h(&J, acc.ptr, sizeof(double));
+        d2h(&J, acc, sizeof(double));
         d2h(&du, peak_out, sizeof(double));
-        if (grad_gamma_out && !grad_on_device) d2h(grad_gamma_out, gg.ptr, cells * sizeof(double));
+        if (grad_gamma_out && !grad_on_device) d2h(grad_gamma_out, args.grad_gamma, cells * sizeof(double));
         sync();
+        block.finished();
         (void)hipEventElapsedTime(&last_forward_ms, e0, e1);
         (void)hipEventElapsedTime(&last_reverse_ms, e1, e2);
         last_forward_steps = forward_steps;
@@ -1090,20 +1101,21 @@ struct cfd_lbm_solver {
         use_device();
         if (!g) throw std::invalid_argument("set_porosity_device needs a device pointer (set_porosity(NULL) clears)");
         const uint64_t blocks = (cells + 255) / 256;
-        DeviceBuffer<unsigned char> fresh, bad;
-        fresh.allocate(cells * real);
-        bad.allocate(sizeof(uint32_t));
-        zero_words(bad.ptr, 1);
-        porosity_from_device<<<static_cast<uint32_t>(blocks), 256, 0, stream>>>(
-            g, fresh.ptr, static_cast<uint32_t>(real), cells, reinterpret_cast<uint32_t*>(bad.ptr));
-        hip_check(hipGetLastError(), "porosity_from_device");
+        if (!reduce_out) reduce_out.allocate(3 * sizeof(double));
+        uint32_t* const bad = reinterpret_cast<uint32_t*>(reduce_out.ptr);
+        zero_words(reduce_out.ptr, 1);
+        check_porosity<<<static_cast<uint32_t>(blocks), 256, 0, stream>>>(g, cells, bad);
+        hip_check(hipGetLastError(), "check_porosity");
         uint32_t n_bad = 0;
-        d2h(&n_bad, bad.ptr, sizeof(n_bad));
+        d2h(&n_bad, bad, sizeof(n_bad));
         sync();
         if (n_bad != 0) throw std::invalid_argument("porosity gamma must lie in [0, 1]");
-        std::swap(gamma.ptr, fresh.ptr);
-        std::swap(gamma.bytes, fresh.bytes);
+        if (!gamma) gamma.allocate(cells * real);
+        porosity_from_device<<<static_cast<uint32_t>(blocks), 256, 0, stream>>>(g, gamma.ptr, static_cast<uint32_t>(real),
+                                                                                cells);
+        hip_check(hipGetLastError(), "porosity_from_device");
         mark_segments();
+        sync();  // the caller's field has been read when this returns
     }
 
     // z-slab halo messages (the slab is this lattice, periodic in z; its neighbours are the slabs
@@ -1582,6 +1594,17 @@ int cfd_lbm_adjoint_run(cfd_lbm_solver* s, uint64_t steps, uint64_t window, uint
         if (checkpoint_every < 1) throw std::invalid_argument("checkpoint interval must be >= 1");
         const double J = need(s).adjoint_run(cfd_hip::kPressureDrop, steps, window, checkpoint_every, 0, x_in, x_out,
                                              grad_gamma, grad_u_peak, nullptr);
+        if (objective) *objective = J;
+    });
+}
+
+int cfd_lbm_adjoint_run_device(cfd_lbm_solver* s, uint64_t steps, uint64_t window, uint64_t checkpoint_every, int x_in,
+                               int x_out, double* objective, double* grad_gamma, double* grad_u_peak, char* error,
+                               size_t cap) {
+    return guarded(error, cap, [&] {
+        if (checkpoint_every < 1) throw std::invalid_argument("checkpoint interval must be >= 1");
+        const double J = need(s).adjoint_run(cfd_hip::kPressureDrop, steps, window, checkpoint_every, 0, x_in, x_out,
+                                             grad_gamma, grad_u_peak, nullptr, true);
         if (objective) *objective = J;
     });
 }

@@ -14,6 +14,7 @@
 // with -ffp-contract=off), so every field except the atomically accumulated two-way particle force
 // is reproducible bit for bit; the global sums (total scalar, volume) are FP64 and deterministic.
 #include "../../include/cfd_lbm/c_api.h"
+#include "device_memory.hpp"
 #include "solver_view.hpp"
 
 #include <hip/hip_runtime.h>
@@ -687,7 +688,7 @@ struct Module {
     void use() const { check(hipSetDevice(flow.device), "hipSetDevice"); }
     float* alloc(uint64_t floats) const {
         void* p = nullptr;
-        check(hipMalloc(&p, floats * sizeof(float)), "hipMalloc");
+        check(cfd_hip::device_malloc(&p, floats * sizeof(float)), "hipMalloc");
         return static_cast<float*>(p);
     }
     void h2d(void* dst, const void* src, size_t bytes) {
@@ -706,7 +707,7 @@ struct Module {
     double sum(const float* v, uint64_t count) {
         if (!partial) {
             void* p = nullptr;
-            check(hipMalloc(&p, (kReduceBlocks + 1) * sizeof(double)), "hipMalloc");
+            check(cfd_hip::device_malloc(&p, (kReduceBlocks + 1) * sizeof(double)), "hipMalloc");
             partial = static_cast<double*>(p);
         }
         sum_partial<<<kReduceBlocks, kBlock, 0, flow.stream>>>(v, count, partial);

@@ -20,6 +20,7 @@
 // equals voxelize.cpp's bit for bit.  Work: (lines x triangles of a tile) u,v tests + (cells x
 // crossings per line) distance tests, instead of cells x triangles.
 #include "voxelize.hpp"
+#include "device_memory.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -297,7 +298,7 @@ __global__ void __launch_bounds__(256) solid_flags(uint8_t* mask, const uint8_t*
 
 template <class T> struct Scratch {
     T* ptr = nullptr;
-    explicit Scratch(size_t n) { check(hipMalloc(reinterpret_cast<void**>(&ptr), std::max<size_t>(n, 1) * sizeof(T)), "hipMalloc"); }
+    explicit Scratch(size_t n) { check(device_malloc(reinterpret_cast<void**>(&ptr), std::max<size_t>(n, 1) * sizeof(T)), "hipMalloc"); }
     ~Scratch() { (void)hipFree(ptr); }
     Scratch(const Scratch&) = delete;
     Scratch& operator=(const Scratch&) = delete;

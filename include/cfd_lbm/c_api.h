@@ -200,6 +200,12 @@ CFD_LBM_API int cfd_lbm_objective_run(cfd_lbm_solver* s, int objective_kind, uin
 CFD_LBM_API int cfd_lbm_adjoint_run(cfd_lbm_solver* s, uint64_t steps, uint64_t window, uint64_t checkpoint_every,
                                     int x_in, int x_out, double* objective, double* grad_gamma, double* grad_u_peak,
                                     char* error, size_t error_capacity);
+/* cfd_lbm_adjoint_run with dJ/dgamma written into DEVICE memory, as
+ * cfd_lbm_adjoint_run_binomial_device does (grad_gamma: cells doubles, 8-byte aligned, required). */
+CFD_LBM_API int cfd_lbm_adjoint_run_device(cfd_lbm_solver* s, uint64_t steps, uint64_t window,
+                                           uint64_t checkpoint_every, int x_in, int x_out, double* objective,
+                                           double* grad_gamma, double* grad_u_peak, char* error,
+                                           size_t error_capacity);
 /* The same with binomial checkpointing: `snapshots` free state buffers besides the start state
  * (0: as many as fit in device memory, 1/16 of it kept free), each step recomputed at most r times
  * where C(snapshots + r, r) >= steps, with the minimal number of forward steps.  objective_kind

@@ -1,0 +1,66 @@
+"""The adjoint's working memory is handed from call to call: runs that find a block another solver's
+run left behind return what a first run returns, bit for bit, and the device-memory gradient of the
+two-level plan is the host one."""
+import numpy as np
+import pytest
+
+from conftest import report
+
+pytestmark = pytest.mark.gpu
+
+
+def _solver(hip, n, storage):
+    from cfd_solvers_amd import geometry
+
+    nx, ny, nz = n
+    s = hip.EsotericPullHipSolver("d3q19", nx, ny, nz, 0.6, storage=storage)
+    flags = geometry.channel_flags(nx, ny, nz, inlet_outlet=True)
+    s.set_flags(flags)
+    s.set_porosity(np.where(flags == 0, 0.004, 0.0).astype(np.float32))
+    s.set_inlet_outlet(0.04, 1.0)
+    return s
+
+
+def _run(s, every, snapshots):
+    s.initialize_uniform()
+    if every:
+        return s.adjoint_run(12, 4, every, 1, s.shape[-1] - 2)
+    return s.adjoint_run_binomial(12, 4, snapshots)[:3]
+
+
+def _same(a, b):
+    return a[0] == b[0] and np.array_equal(a[1], b[1]) and a[2] == b[2]
+
+
+@pytest.mark.parametrize("storage", ["fp32", "fp16s"])
+def test_reused_blocks_change_nothing(hip, storage):
+    plans = [(4, 0), (0, 3), (5, 0), (0, 2)]
+    # Each shape's first result comes from a process state in which its solver is the only one, so
+    # that the pool is empty when it starts.
+    shapes = [(19, 14, 12), (33, 12, 11)]
+    first = {}
+    for n in shapes:
+        for plan in plans:
+            report("workspace_first", storage=storage, n=n, plan=plan)
+            s = _solver(hip, n, storage)
+            first[n, plan] = _run(s, *plan)
+            s.close()
+    solvers = {n: _solver(hip, n, storage) for n in shapes}
+    for plan in plans:
+        for n in shapes:
+            report("workspace_again", storage=storage, n=n, plan=plan)
+            assert _same(_run(solvers[n], *plan), first[n, plan])
+
+
+def test_device_gradient_of_the_two_level_plan(hip, dev):
+    n = (19, 14, 12)
+    s = _solver(hip, n, "fp32")
+    want = _run(s, 4, 0)
+    grad = dev.upload(np.full(s.cells, np.nan))
+    report("two_level_device", n=n)
+    s.initialize_uniform()
+    J, du = s.adjoint_run_device(12, 4, 4, grad)
+    assert J == want[0] and du == want[2]
+    assert np.array_equal(dev.download(grad, s.shape, np.float64), want[1])
+    with pytest.raises(RuntimeError, match="aligned"):
+        s.adjoint_run_device(12, 4, 4, 0)
