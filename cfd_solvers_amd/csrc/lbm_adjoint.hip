@@ -192,7 +192,7 @@ __device__ __forceinline__ Real plane_weight(const AdjointArgs& a, uint32_t x, b
 
 // One transposed step at the given parity, in place on lam.  fstate holds the forward state f_t.
 template <int Q, class T, bool Odd, bool Bounded>
-__global__ __launch_bounds__(256) void adjoint_step(const void* __restrict__ fstate, void* __restrict__ lam_buf,
+__global__ __launch_bounds__(kStepThreads<typename Storage<T>::Real>) void adjoint_step(const void* __restrict__ fstate, void* __restrict__ lam_buf,
                                                     const Geometry g, const Physics<typename Storage<T>::Real> p,
                                                     const AdjointArgs a) {
     using Real = typename Storage<T>::Real;
@@ -463,8 +463,8 @@ template <int Q, class T> struct AdjOps final : AdjointOps {
     void step(const LaunchState& st, bool odd, bool bounded, const void* fstate, void* lam,
               const AdjointArgs& a) const override {
         per_parity(odd, bounded, [&](auto O, auto B) {
-            hipLaunchKernelGGL((adjoint_step<Q, T, decltype(O)::value, decltype(B)::value>), grid(st.geo),
-                               block(st.geo), st.adjoint_lds, st.stream, fstate, lam, st.geo,
+            hipLaunchKernelGGL((adjoint_step<Q, T, decltype(O)::value, decltype(B)::value>), grid_of(st.step_geo),
+                               block_of(st.step_geo), st.adjoint_lds, st.stream, fstate, lam, st.step_geo,
                                *static_cast<const Physics<Real>*>(st.physics), a);
         });
         check(hipGetLastError(), "adjoint_step launch");

@@ -110,7 +110,7 @@ struct cfd_lbm_solver {
     size_t nx = 0, ny = 0, nz = 0, cells = 0;
     float tau = 0.6F, ax = 0, ay = 0, az = 0;
     size_t elem = 4, real = 4;
-    Geometry geo{};
+    Geometry geo{}, step_geo{};
     hipStream_t stream = nullptr;
     const KernelOps* ops = nullptr;
     DeviceBuffer<unsigned char> f, flags, links, link_vel, segments, solid_rho, gamma, lacc, macro, partial, reduce_out;
@@ -151,28 +151,13 @@ struct cfd_lbm_solver {
         elem = storage == 1 ? 2 : (storage == 2 || storage == 4 ? 8 : 4);
         real = storage == 2 || storage == 4 ? 8 : 4;
 
-        // Launch geometry: 256-thread tiles, bx a power of two in [64, 256] covering x, so that a
-        // wavefront's 64 lanes lie in one row segment (the bounded step reads the segment's span
-        // once per wavefront).
+        // Launch geometry: 256-thread tiles, bx a power of two in [64, 256] covering x.
         uint32_t bx = 64;
         while (bx < nx && bx < 256) bx <<= 1;
-        if (const char* v = std::getenv("CFD_LBM_BX")) {  // tuning: tile width 64, 128 or 256
-            const long w = std::atol(v);
-            if (w == 64 || w == 128 || w == 256) bx = static_cast<uint32_t>(w);
-        }
         geo.nx = static_cast<uint32_t>(nx);
         geo.ny = static_cast<uint32_t>(ny);
         geo.nz = static_cast<uint32_t>(nz);
-        geo.bx = bx;
-        geo.by = 256U / bx;
-        geo.tiles_x = static_cast<uint32_t>((nx + bx - 1) / bx);
-        geo.tiles_y = static_cast<uint32_t>((ny + geo.by - 1) / geo.by);
-        const uint64_t tiles = static_cast<uint64_t>(geo.tiles_x) * geo.tiles_y * nz;
-        if (tiles >= (uint64_t{1} << 31)) throw std::invalid_argument("lattice too large for one launch");
-        geo.tiles = static_cast<uint32_t>(tiles);
-        geo.xcd_remap = 0U;
-        if (const char* v = std::getenv("CFD_LBM_XCD_REMAP"))
-            geo.xcd_remap = (std::atoi(v) != 0 && geo.tiles % 8U == 0U && geo.tiles >= 64U) ? 1U : 0U;
+        tile_geometry(geo, bx, 256U / bx);
         // Population layout (Geometry in lbm_device.hpp).  Kernels address a population as a plane
         // base plus a 32-bit byte offset, reaching one plane further for bounce-back; the adjoint
         // keeps lambda in the same layout with `real`-sized elements.  Blocks of 2^k x-rows holding
@@ -212,6 +197,10 @@ struct cfd_lbm_solver {
             if (2U * geo.stride * elem > (uint64_t{1} << 32))
                 throw std::invalid_argument("lattice too large: two population planes must fit in 4 GiB");
         }
+        step_geo = geo;
+        const uint32_t width = step_width();
+        tile_geometry(step_geo, width, width < 256U ? 256U / width : 1U);
+        step_geo.xcd_group = xcd_group();
         // Resident wavefronts per SIMD of the step kernel, bounded and periodic, capped by reserving
         // LDS per block (160 KiB per CU; a 256-thread block puts one wave on each of the 4 SIMDs).
         // Measured on MI355X:
@@ -233,7 +222,13 @@ struct cfd_lbm_solver {
             waves_bounded = waves_periodic = 5;
         }
         if (const char* v = std::getenv("CFD_LBM_WAVES")) waves_bounded = waves_periodic = std::atol(v);
-        auto lds_cap = [](long w) { return w >= 3 && w < 8 ? static_cast<uint32_t>(163840 / w - 1024) : 0U; };
+        // A block of `threads` threads is threads / 256 wavefronts on each SIMD.
+        const long threads = static_cast<long>(step_geo.bx) * step_geo.by;
+        auto lds_cap = [threads](long w) {
+            if (w < 3 || w >= 8) return 0U;
+            const long blocks = std::max(1L, (w * 256 + threads / 2) / threads);
+            return static_cast<uint32_t>(std::min(163840 / blocks - 1024, 65536L));
+        };
         step_lds = lds_cap(waves_bounded);
         step_lds_periodic = lds_cap(waves_periodic);
         // The transposed step (adjoint) runs 6 (FP16) or 5 (FP32) waves per SIMD by its registers.
@@ -270,6 +265,64 @@ struct cfd_lbm_solver {
             (void)hipStreamDestroy(stream);
         }
         cfd_hip::WorkspacePool::instance().leave();
+    }
+
+    static void tile_geometry(Geometry& g, uint32_t bx, uint32_t by) {
+        g.bx = bx;
+        g.by = by;
+        g.tiles_x = (g.nx + bx - 1U) / bx;
+        g.tiles_y = (g.ny + by - 1U) / by;
+        const uint64_t tiles = static_cast<uint64_t>(g.tiles_x) * g.tiles_y * g.nz;
+        if (tiles >= (uint64_t{1} << 31)) throw std::invalid_argument("lattice too large for one launch");
+        g.tiles = static_cast<uint32_t>(tiles);
+        g.xcd_group = 0U;
+    }
+
+    // Width of a step tile.  Neighbouring tiles of a row share cache lines at their common edge
+    // (populations are read and written at x - 1, x and x + 1), so a tile spans the row where a block
+    // can (256^3 cavity: 454 us a step with 256-wide tiles, 484 with 128, 563 with 64), and it launches
+    // no whole wavefronts beyond the row's end: five to eight 64-cell segments are one tile of just
+    // that width (301 x 150 x 141 FP32S: 190 us against 252 with 256-wide tiles, 203 with 128; 350 wide
+    // FP32: 216 against 287; 270 wide: 169 against 240).  Up to four segments take the 256-thread tile
+    // (192 wide, 192^3 FP32: 191 us with a 192-thread tile, 187 with 256).  Longer rows take the width
+    // that launches least, 256 unless that adds more than 1/8 to the row (2-D, 1100 wide: 25.4 us with
+    // 256, 26.1-27.4 with 320-512).  FP64 needs the registers of a 256-thread block, so its rows of
+    // more than four segments take 128 where that launches fewer (260 wide: 309 us against 405).
+    uint32_t step_width() const {
+        const uint32_t most = real == 8 ? 4U : 8U;  // kStepThreads / 64
+        if (const char* v = std::getenv("CFD_LBM_BX")) {  // tuning: 64, 128 or a multiple of 64 up to the most
+            const long w = std::atol(v);
+            if (w >= 64 && w <= 64 * static_cast<long>(most) && w % 64 == 0 && w != 192) return static_cast<uint32_t>(w);
+        }
+        const uint32_t segments_x = seg_x();
+        const auto launched = [segments_x](uint32_t w) { return (segments_x + w - 1U) / w * w; };
+        if (segments_x <= 4U) return geo.bx;
+        if (segments_x <= most) return 64U * segments_x;
+        if (real == 8) return launched(2U) < launched(4U) ? 128U : 256U;
+        if (launched(4U) * 8U <= segments_x * 9U) return 256U;
+        uint32_t best = 4U;
+        for (uint32_t w = 5U; w <= most; ++w)
+            if (launched(w) < launched(best)) best = w;
+        return 64U * best;
+    }
+
+    // Consecutive tiles of one XCD in the step kernels.  A lattice that fits the 256 MiB Infinity Cache
+    // gives each XCD one run of rows: its L2 then holds the lines that neighbouring rows share, and a
+    // line written in parts is completed in one L2 (D3Q27 56^3: 7.4 us a step against 10.8 round-robin;
+    // D3Q19 FP16S 150^3: 42 against 59; D3Q19 FP32 128^3 cavity: 49.5 against 54.6; D2Q9 600^2: 6.4
+    // against 9.4).  On larger lattices long runs cost HBM locality (512^2 x 256 FP16S: 1099 us in one
+    // run each, 1005 round-robin), and only rows that are not whole 128-byte lines share lines: runs of
+    // 8 tiles there (D3Q27 200^3: 324 us against 364; 190 x 150 x 141 FP32S: 111 against 122), single
+    // tiles elsewhere (4096^2 D2Q9: 203 us against 211 in runs of 8).
+    uint32_t xcd_group() const {
+        const uint32_t run = (step_geo.tiles + 7U) / 8U;
+        if (const char* v = std::getenv("CFD_LBM_XCD_REMAP")) {  // tuning: 0 round-robin, 1 one run each, n: n tiles
+            const long g = std::atol(v);
+            return g <= 0 ? 0U : (g == 1 ? run : static_cast<uint32_t>(std::min<long>(g, run)));
+        }
+        if (step_geo.tiles > (1U << 22)) return 0U;  // the padding to whole runs stays far below the grid's limit
+        if (pop_elems * elem <= (uint64_t{256} << 20)) return run;
+        return nx * elem % 128U != 0 ? std::min(8U, run) : 0U;
     }
 
     void use_device() const { hip_check(hipSetDevice(device), "hipSetDevice"); }
@@ -310,7 +363,7 @@ struct cfd_lbm_solver {
     LaunchState state() {
         if (real == 8) build_physics<double>();
         else build_physics<float>();
-        return LaunchState{f.ptr, geo, physics, stream, static_cast<uint32_t>(cells), step_lds, step_lds_periodic,
+        return LaunchState{f.ptr, geo, step_geo, physics, stream, static_cast<uint32_t>(cells), step_lds, step_lds_periodic,
                            adjoint_lds};
     }
 

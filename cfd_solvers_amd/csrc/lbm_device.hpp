@@ -190,11 +190,11 @@ template <class S, int Q, int D, class Real> __device__ __forceinline__ Real sta
 }
 
 // ------------------------------------------------------------------ launch geometry
-// A block is a bx*by = 256-thread tile of one z plane (bx spans x: 64, 128 or 256, so that the 64
-// lanes of a wavefront lie in one row and one 64-cell row segment).  Tiles are
-// numbered x-fastest.  The hardware deals consecutive blocks round-robin to the 8 XCDs, so the
-// chip streams through neighbouring rows together; xcd_remap (off by default: it measured slower
-// on MI355X) instead gives each XCD one contiguous slab of tiles.
+// A block is a bx*by tile of one z plane (bx spans x, a multiple of 64, so that the 64 lanes of a
+// wavefront lie in one row and one 64-cell row segment): 256 threads in the kernels that reduce over a
+// block, 64 to 512 in the step kernels.  Tiles are numbered x-fastest.  The hardware deals
+// consecutive blocks round-robin to the 8 XCDs; with xcd_group != 0 each XCD instead gets runs of
+// xcd_group consecutive tiles, so that the cache lines which neighbouring tiles share stay in one L2.
 // Population layout.  The lattice's x-rows (row r = z*ny + y) are grouped into blocks of 2^row_shift
 // consecutive rows; a block holds the q direction planes of its cells one after another, `stride`
 // elements apart, and blocks are `block_elems` elements apart.  Slot (d, cell (r, x)) is element
@@ -206,7 +206,7 @@ struct Geometry {
     uint32_t nx, ny, nz;
     uint32_t bx, by;
     uint32_t tiles_x, tiles_y, tiles;
-    uint32_t xcd_remap;
+    uint32_t xcd_group;    // consecutive tiles of one XCD, 0: single tiles round-robin
     uint32_t row_shift;    // log2 rows per block; 31: one block (plain planes)
     uint32_t block_elems;  // elements per block (q * stride); unused when row_shift = 31
     uint64_t stride;       // elements between consecutive direction planes of a block
@@ -219,7 +219,12 @@ __host__ __device__ __forceinline__ uint32_t row_base(const Geometry& g, uint32_
 
 __device__ __forceinline__ bool cell_coords(const Geometry& g, uint32_t& x, uint32_t& y, uint32_t& z) {
     uint32_t b = blockIdx.x;
-    if (g.xcd_remap) b = (b & 7U) * (g.tiles >> 3) + (b >> 3);
+    if (g.xcd_group != 0U) {
+        const uint32_t k = b >> 3;  // the how manyeth block of its XCD
+        const uint32_t run = k / g.xcd_group;
+        b = (8U * run + (b & 7U)) * g.xcd_group + (k - run * g.xcd_group);
+        if (b >= g.tiles) return false;
+    }
     const uint32_t tx = b % g.tiles_x;
     const uint32_t r = b / g.tiles_x;
     const uint32_t ty = r % g.tiles_y;

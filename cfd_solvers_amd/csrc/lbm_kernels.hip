@@ -42,8 +42,8 @@ __device__ __forceinline__ void update_cell(const void* src, void* dst, const Ge
 // In place when src == dst (the time step); src != dst writes the next state into another buffer
 // (recomputation of stored states for the adjoint).  Every slot the next step reads is written.
 template <int Q, class T, bool Odd, bool Bounded, bool Forced>
-__global__ __launch_bounds__(256) CFD_LBM_OCCUPANCY void stream_collide(const void* src, void* dst, const Geometry g,
-                                                                        const Physics<typename Storage<T>::Real> p) {
+__global__ __launch_bounds__(kStepThreads<typename Storage<T>::Real>) CFD_LBM_OCCUPANCY void stream_collide(
+    const void* src, void* dst, const Geometry g, const Physics<typename Storage<T>::Real> p) {
     uint32_t x, y, z;
     if (!cell_coords(g, x, y, z)) return;
     const Neighbourhood h = neighbourhood(g, x, y, z);
@@ -365,7 +365,7 @@ __global__ __launch_bounds__(256) void thaw_walls(void* __restrict__ f, const Ge
 
 // ------------------------------------------------------------------ macroscopic fields
 template <int Q, class T, bool Odd, bool Bounded>
-__global__ __launch_bounds__(256) void macroscopic(const void* __restrict__ f, const Geometry g,
+__global__ __launch_bounds__(kStepThreads<typename Storage<T>::Real>) void macroscopic(const void* __restrict__ f, const Geometry g,
                                                    const Physics<typename Storage<T>::Real> p,
                                                    typename Storage<T>::Real* __restrict__ out) {
     using Real = typename Storage<T>::Real;
@@ -645,16 +645,15 @@ inline void check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-inline dim3 block_of(const Geometry& g) { return dim3(g.bx, g.by, 1); }
-inline dim3 grid_of(const Geometry& g) { return dim3(g.tiles, 1, 1); }
 
 template <int Q, class T> struct Ops final : KernelOps {
     using Real = typename Storage<T>::Real;
 
     template <bool Odd, bool Bounded, bool Forced>
     static void step_t(const LaunchState& st, const void* src, void* dst) {
-        hipLaunchKernelGGL((stream_collide<Q, T, Odd, Bounded, Forced>), grid_of(st.geo), block_of(st.geo),
-                           Bounded ? st.step_lds : st.step_lds_periodic, st.stream, src, dst, st.geo,
+        hipLaunchKernelGGL((stream_collide<Q, T, Odd, Bounded, Forced>), grid_of(st.step_geo),
+                           block_of(st.step_geo), Bounded ? st.step_lds : st.step_lds_periodic, st.stream, src, dst,
+                           st.step_geo,
                            *static_cast<const Physics<Real>*>(st.physics));
     }
     void step(const LaunchState& st, bool odd, bool bounded, bool forced, const void* src, void* dst) const override {
@@ -723,8 +722,8 @@ template <int Q, class T> struct Ops final : KernelOps {
     }
     void macroscopic(const LaunchState& st, bool odd, bool bounded, void* out) const override {
         per_parity(st, odd, bounded, [&](auto O, auto B) {
-            hipLaunchKernelGGL((cfd_hip::macroscopic<Q, T, decltype(O)::value, decltype(B)::value>), grid_of(st.geo),
-                               block_of(st.geo), 0, st.stream, st.f, st.geo,
+            hipLaunchKernelGGL((cfd_hip::macroscopic<Q, T, decltype(O)::value, decltype(B)::value>),
+                               grid_of(st.step_geo), block_of(st.step_geo), 0, st.stream, st.f, st.step_geo,
                                *static_cast<const Physics<Real>*>(st.physics), static_cast<Real*>(out));
         });
         check(hipGetLastError(), "macroscopic launch");

@@ -12,7 +12,8 @@ namespace cfd_hip {
 
 struct LaunchState {
     void* f;                 // population planes
-    Geometry geo;
+    Geometry geo;            // 256-thread tiles: setup, probes and reductions
+    Geometry step_geo;       // the step kernels' tiles (forward, transposed, macroscopic)
     const void* physics;     // Physics<float> or Physics<double> (host copy, passed by value)
     hipStream_t stream;
     uint32_t cells;
@@ -20,6 +21,16 @@ struct LaunchState {
     uint32_t step_lds_periodic;  // the same for the periodic step
     uint32_t adjoint_lds;    // the same for the transposed step
 };
+
+inline dim3 block_of(const Geometry& g) { return dim3(g.bx, g.by, 1); }
+inline dim3 grid_of(const Geometry& g) {
+    if (g.xcd_group == 0U) return dim3(g.tiles, 1, 1);
+    const uint32_t round = 8U * g.xcd_group;  // at most 2^31 / 8 + 8 tiles: no overflow
+    return dim3((g.tiles + round - 1U) / round * round, 1, 1);
+}
+
+// Most threads of a step block.  The FP64 kernels need more registers than 512 threads leave each.
+template <class Real> constexpr int kStepThreads = sizeof(Real) == 8 ? 256 : 512;
 
 // One instance per (lattice, storage); every launch is asynchronous on st.stream.
 struct KernelOps {
