@@ -23,7 +23,7 @@ PROBE = PKG / "libhbm_probe.so"
 APPS = {"cfd-bench": PKG / "apps" / "cfd_bench.cpp", "cfd-solve": PKG / "apps" / "cfd_solve.cpp",
         "cfd-distributed": PKG / "apps" / "cfd_distributed.cpp"}
 
-HIP_SOURCES = ["lbm_kernels.hip", "lbm_adjoint.hip", "voxelize.hip", "multiphysics.hip", "lbm_capi.hip"]
+HIP_SOURCES = ["lbm_kernels.hip", "lbm_tiled.hip", "lbm_adjoint.hip", "voxelize.hip", "multiphysics.hip", "lbm_capi.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -10,6 +10,7 @@
 #include "device_memory.hpp"
 #include "lbm_adjoint.hpp"
 #include "lbm_kernels.hpp"
+#include "lbm_tiled.hpp"
 #include "solver_view.hpp"
 #include "voxelize.hpp"
 
@@ -122,6 +123,11 @@ struct cfd_lbm_solver {
     std::vector<uint8_t> host_flags;  // copy of the flags (empty: periodic)
     float last_forward_ms = 0.0F, last_reverse_ms = 0.0F;
     uint64_t last_forward_steps = 0;
+    // The second lattice of the several-steps-per-launch kernels, taken at the first call that uses
+    // them and held until the solver goes; the state is in `f` between calls.
+    unsigned char* second = nullptr;
+    size_t second_bytes = 0;
+    bool second_refused = false;
     mutable TransferStats stats;
     // Host copy of the Physics<Real> passed by value to every launch.
     alignas(16) unsigned char physics[sizeof(Physics<double>)] = {};
@@ -264,6 +270,7 @@ struct cfd_lbm_solver {
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
         }
+        if (second) cfd_hip::WorkspacePool::instance().put(second, second_bytes, true);
         cfd_hip::WorkspacePool::instance().leave();
     }
 
@@ -1231,19 +1238,53 @@ struct cfd_lbm_solver {
         hip_check(hipGetLastError(), "zero_words");
     }
 
+    // Whether `count` steps may run several to a launch (lbm_tiled.hip): an unporous D2Q9 lattice whose
+    // second copy is within the workspace bound, outside of stream capture (a graph is replayed on
+    // `f` alone, and it must not hold an allocation).
+    bool several_per_launch(uint64_t count) {
+        if (count < 4U || gamma || second_refused || !cfd_hip::tiled_supported(q, storage, nx, ny)) return false;
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+        if (second) return true;
+        size_t free_b = 0, total = 0;
+        hip_check(hipMemGetInfo(&free_b, &total), "hipMemGetInfo");
+        second_refused = f.bytes > total / cfd_hip::WorkspacePool::kKeptFraction;
+        if (second_refused) return false;
+        try {
+            second = cfd_hip::WorkspacePool::instance().take(f.bytes, &second_bytes);
+        } catch (const std::runtime_error&) {  // no room: the single step needs none
+            (void)hipGetLastError();
+            second_refused = true;
+        }
+        return second != nullptr;
+    }
+
     void step(uint64_t count) {
         use_device();
         const bool b = bounded();
         const bool forced = ax != 0.0F || ay != 0.0F || az != 0.0F || static_cast<bool>(lacc) || les;
         LaunchState st = state();
-        for (uint64_t k = 0; k < count; ++k) {
+        const auto single = [&] {
             ops->step(st, odd(), b, forced, f.ptr, f.ptr);
             ++t;
+            --count;
+        };
+        if (several_per_launch(count - (odd() && count > 0 ? 1U : 0U))) {
+            if (odd()) single();  // the tiled kernels start at even parity
+            // Pairs of launches, f to the second lattice and back.
+            for (int k = 4; k >= 2; k -= 2)
+                for (; count >= 2U * static_cast<uint64_t>(k); count -= 2U * static_cast<uint64_t>(k)) {
+                    cfd_hip::tiled_steps(storage, st, k, b, forced, f.ptr, second);
+                    cfd_hip::tiled_steps(storage, st, k, b, forced, second, f.ptr);
+                    t += 2U * static_cast<uint64_t>(k);
+                }
         }
+        while (count > 0) single();
     }
 
     float step_timed(uint64_t count) {
         use_device();
+        (void)several_per_launch(count);  // its allocation is not part of the steps
         TimingEvent e0, e1;
         float ms = 0.0F;
         hip_check(hipEventRecord(e0.e, stream), "hipEventRecord");
@@ -1338,7 +1379,7 @@ struct cfd_lbm_solver {
     size_t population_bytes() const { return static_cast<size_t>(q) * cells * elem; }
     size_t resident_bytes() const {
         return f.bytes + flags.bytes + links.bytes + link_vel.bytes + segments.bytes + solid_rho.bytes + gamma.bytes + lacc.bytes + macro.bytes + partial.bytes +
-               reduce_out.bytes;
+               reduce_out.bytes + second_bytes;
     }
 };
 

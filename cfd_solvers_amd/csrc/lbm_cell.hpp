@@ -92,6 +92,39 @@ template <class S, class Real> __device__ __forceinline__ Real wall_term(Real v)
     else return v;
 }
 
+// Moving walls: a population bounced off a wall of velocity u_w is stored as f - 6 w rho_w (c . u_w),
+// the push form of src/lbm/d2q9.cpp:217-223.  Only cells next to a moving wall read their per-link
+// wall-velocity indices.
+template <int Q, class S, class Real>
+__device__ __forceinline__ void moving_wall_terms(const Physics<Real>& p, uint32_t desc, uint32_t n, Real rho,
+                                                  Real (&fout)[Q]) {
+    using L = Lattice<Q>;
+    if ((desc >> kMovingBit) & 1U) {
+        constexpr int kW = PairSlots<Q>::kVelWords;
+        uint32_t vel[kW];
+        for (int w = 0; w < kW; ++w) vel[w] = p.link_vel[static_cast<uint64_t>(n) * kW + w];
+        const Real rho_wall = rho > Real(1.0e-8) ? rho : Real(1.0e-8);
+        static_for<(Q - 1) / 2>([&](auto P) {
+            constexpr int i = 2 * decltype(P)::value + 1;
+            // fout[i] travels to dn = n + c_i (link i); fout[i+1] to up = n - c_i (link i-1).
+            const uint32_t ka = (vel[i / 10] >> (3 * (i % 10))) & 7U;
+            if (ka != 0U) {
+                const Real cu = static_cast<Real>(L::cx[i]) * p.wall_u[ka][0] +
+                                static_cast<Real>(L::cy[i]) * p.wall_u[ka][1] +
+                                static_cast<Real>(L::cz[i]) * p.wall_u[ka][2];
+                fout[i] = fout[i] - wall_term<S>(Real(6) * lattice_weight<S, Q, i, Real>() * rho_wall * cu);
+            }
+            const uint32_t kb = (vel[(i - 1) / 10] >> (3 * ((i - 1) % 10))) & 7U;
+            if (kb != 0U) {
+                const Real cu = static_cast<Real>(L::cx[i + 1]) * p.wall_u[kb][0] +
+                                static_cast<Real>(L::cy[i + 1]) * p.wall_u[kb][1] +
+                                static_cast<Real>(L::cz[i + 1]) * p.wall_u[kb][2];
+                fout[i + 1] = fout[i + 1] - wall_term<S>(Real(6) * lattice_weight<S, Q, i + 1, Real>() * rho_wall * cu);
+            }
+        });
+    }
+}
+
 template <int Q, class T, bool Odd, bool Bounded>
 __device__ __forceinline__ void store_cell(void* f, const Geometry& g, const Physics<typename Storage<T>::Real>& p,
                                            uint32_t n, uint32_t x, uint32_t y, uint32_t z,
@@ -99,36 +132,7 @@ __device__ __forceinline__ void store_cell(void* f, const Geometry& g, const Phy
                                            const PairSlots<Q>& s) {
     using L = Lattice<Q>;
     using S = Storage<T>;
-    using Real = typename Storage<T>::Real;
-    if constexpr (Bounded) {
-        if ((s.desc >> kMovingBit) & 1U) {
-            // Moving wall: a population bounced off a wall of velocity u_w is stored as
-            // f - 6 w rho_w (c . u_w), the push form of src/lbm/d2q9.cpp:217-223.  Only cells next
-            // to a moving wall come here; they read their per-link wall-velocity indices.
-            constexpr int kW = PairSlots<Q>::kVelWords;
-            uint32_t vel[kW];
-            for (int w = 0; w < kW; ++w) vel[w] = p.link_vel[static_cast<uint64_t>(n) * kW + w];
-            const Real rho_wall = rho > Real(1.0e-8) ? rho : Real(1.0e-8);
-            static_for<(Q - 1) / 2>([&](auto P) {
-                constexpr int i = 2 * decltype(P)::value + 1;
-                // fout[i] travels to dn = n + c_i (link i); fout[i+1] to up = n - c_i (link i-1).
-                const uint32_t ka = (vel[i / 10] >> (3 * (i % 10))) & 7U;
-                if (ka != 0U) {
-                    const Real cu = static_cast<Real>(L::cx[i]) * p.wall_u[ka][0] +
-                                    static_cast<Real>(L::cy[i]) * p.wall_u[ka][1] +
-                                    static_cast<Real>(L::cz[i]) * p.wall_u[ka][2];
-                    fout[i] = fout[i] - wall_term<S>(Real(6) * lattice_weight<S, Q, i, Real>() * rho_wall * cu);
-                }
-                const uint32_t kb = (vel[(i - 1) / 10] >> (3 * ((i - 1) % 10))) & 7U;
-                if (kb != 0U) {
-                    const Real cu = static_cast<Real>(L::cx[i + 1]) * p.wall_u[kb][0] +
-                                    static_cast<Real>(L::cy[i + 1]) * p.wall_u[kb][1] +
-                                    static_cast<Real>(L::cz[i + 1]) * p.wall_u[kb][2];
-                    fout[i + 1] = fout[i + 1] - wall_term<S>(Real(6) * lattice_weight<S, Q, i + 1, Real>() * rho_wall * cu);
-                }
-            });
-        }
-    }
+    if constexpr (Bounded) moving_wall_terms<Q, S>(p, s.desc, n, rho, fout);
     const uint32_t off_n = opaque_offset(s.self);
     store_at<T>(plane<T>(f, g, 0), off_n, S::template encode<Q, 0>(fout[0]));
     static_for<(Q - 1) / 2>([&](auto P) {

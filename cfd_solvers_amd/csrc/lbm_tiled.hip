@@ -1,0 +1,209 @@
+// lbm_tiled.hip -- several D2Q9 time steps in one launch, on tiles held in LDS.
+//
+// A single in-place step reads and writes every population once, so a large 2-D lattice is bound by
+// HBM and a small one by the launch.  Here a block loads a tile with a halo of K cells, takes K steps
+// on it in LDS and writes the interior into a second lattice array (the halo cells' old state is
+// read by several blocks, so the result cannot overwrite it).  The halo is recomputed: level s (1..K)
+// updates the cells at least s away from the tile's edge.
+//
+// The tile is kept in the lattice's own esoteric slot map: level 1 loads from the global slots and
+// stores into LDS slots, the levels between work in place on LDS (each slot is read and written by one
+// cell, so one barrier a level is enough and nothing is double-buffered), level K stores to the global
+// slots.  Every level rounds to the storage type and uses the step kernel's arithmetic, so K steps here
+// are K single steps bit for bit, the slots left behind at walls included.
+#include "lbm_tiled.hpp"
+#include "lbm_cell.hpp"
+
+#include <hip/hip_runtime.h>
+
+#include <stdexcept>
+#include <string>
+
+namespace cfd_hip {
+
+namespace {
+
+constexpr int Q = 9;
+
+// Populations of the cell at LDS slot `c` (Odd: parity of the step), and back.
+template <class T, bool Odd, bool Bounded, int W, int P>
+__device__ __forceinline__ void load_tile(const T* t, int c, uint32_t desc, typename Storage<T>::Real (&f)[Q]) {
+    using L = Lattice<Q>;
+    using S = Storage<T>;
+    f[0] = S::template decode<Q, 0>(t[c]);
+    static_for<(Q - 1) / 2>([&](auto PP) {
+        constexpr int i = 2 * decltype(PP)::value + 1;
+        constexpr int up = -(L::cy[i] * W + L::cx[i]);
+        if constexpr (Bounded) {
+            const bool wup = ((desc >> (i - 1)) & 1U) != 0U, wdn = ((desc >> i) & 1U) != 0U;
+            f[i] = S::template decode<Q, i>(t[c + up + (Odd != wup ? i + 1 : i) * P]);
+            f[i + 1] = S::template decode<Q, i + 1>(t[c + (Odd != wdn ? i : i + 1) * P]);
+        } else {
+            f[i] = S::template decode<Q, i>(t[c + up + (Odd ? i + 1 : i) * P]);
+            f[i + 1] = S::template decode<Q, i + 1>(t[c + (Odd ? i : i + 1) * P]);
+        }
+    });
+}
+template <class T, bool Odd, int W, int P>
+__device__ __forceinline__ void store_tile(T* t, int c, const typename Storage<T>::Real (&f)[Q]) {
+    using L = Lattice<Q>;
+    using S = Storage<T>;
+    t[c] = S::template encode<Q, 0>(f[0]);
+    static_for<(Q - 1) / 2>([&](auto PP) {
+        constexpr int i = 2 * decltype(PP)::value + 1;
+        constexpr int up = -(L::cy[i] * W + L::cx[i]);
+        t[c + (Odd ? i : i + 1) * P] = S::template encode<Q, i>(f[i]);
+        t[c + up + (Odd ? i + 1 : i) * P] = S::template encode<Q, i + 1>(f[i + 1]);
+    });
+}
+
+// All K levels of one tile: W x H slots in LDS, the thread's column rx, rows ry0, ry0 + Rows, ...;
+// `w` x `h` of them lie within the lattice's last cell and its halo.
+template <class T, bool Bounded, bool Forced, int K, int W, int H, int Rows>
+__device__ __forceinline__ void advance_tile(const void* src, void* dst, const Geometry& g,
+                                             const Physics<typename Storage<T>::Real>& p, T* t, int rx, int ry0,
+                                             uint32_t x, int y_first, int w, int h) {
+    using Real = typename Storage<T>::Real;
+    using S = Storage<T>;
+    constexpr int P = W * H;
+    static_for<K>([&](auto LL) {
+        constexpr int s = decltype(LL)::value + 1;
+        constexpr bool Odd = (s & 1) == 0;  // the tile starts at even parity
+        if (rx >= s && rx < w - s)
+            for (int ry = ry0 + s; ry < h - s; ry += Rows) {
+                int yy = y_first + ry;  // -K .. ny + K - 1
+                if (yy < 0) yy += static_cast<int>(g.ny);
+                if (yy >= static_cast<int>(g.ny)) yy -= static_cast<int>(g.ny);
+                const uint32_t y = static_cast<uint32_t>(yy);
+                const uint32_t n = y * g.nx + x;
+                uint32_t desc = 0U;
+                if constexpr (Bounded) desc = p.links[n];
+                const uint32_t type = (desc >> kTypeShift) & 3U;
+                if (Bounded && type == kTypeWall) continue;
+                const int c = ry * W + rx;
+                Real f[Q];
+                if constexpr (s == 1) {
+                    PairSlots<Q> slots;
+                    load_cell<Q, T, Odd, Bounded>(src, g, desc, neighbourhood(g, x, y, 0U), f, slots);
+                } else {
+                    load_tile<T, Odd, Bounded, W, P>(t, c, desc, f);
+                }
+                [[maybe_unused]] Real fin[Q];
+                if constexpr (Bounded && s == K)
+                    static_for<Q>([&](auto DD) { fin[decltype(DD)::value] = f[decltype(DD)::value]; });
+                const Real rho = collide<Q, Forced, S>(p, static_cast<const Real*>(nullptr), g,
+                                                       static_cast<uint8_t>(type), n, y, 0U, f);
+                if constexpr (s < K) {
+                    if constexpr (Bounded) moving_wall_terms<Q, S>(p, desc, n, rho, f);
+                    store_tile<T, Odd, W, P>(t, c, f);
+                } else {
+                    const Neighbourhood nb = neighbourhood(g, x, y, 0U);
+                    PairSlots<Q> slots;
+                    slots.self = nb.cell(0, 0, 0) * static_cast<uint32_t>(sizeof(T));
+                    slots.desc = desc;
+                    static_for<(Q - 1) / 2>([&](auto PP) {
+                        constexpr int i = 2 * decltype(PP)::value + 1;
+                        using L = Lattice<Q>;
+                        slots.up[i] = nb.cell(-L::cx[i], -L::cy[i], 0) * static_cast<uint32_t>(sizeof(T));
+                        // A wall link's population was read from the slot of the other parity, which the
+                        // in-place step leaves as it was.
+                        if constexpr (Bounded) {
+                            if (slots.is_wall_link(i - 1))
+                                store_at<T>(plane<T>(dst, g, Odd ? i : i + 1), slots.up[i],
+                                            S::template encode<Q, i>(fin[i]));
+                            if (slots.is_wall_link(i))
+                                store_at<T>(plane<T>(dst, g, Odd ? i + 1 : i), slots.self,
+                                            S::template encode<Q, i + 1>(fin[i + 1]));
+                        }
+                    });
+                    store_cell<Q, T, Odd, Bounded>(dst, g, p, n, x, y, 0U, rho, f, slots);
+                }
+            }
+        if constexpr (s < K) __syncthreads();
+    });
+}
+
+template <class T, bool Bounded, bool Forced, int K, int W, int H, int Rows>
+__global__ __launch_bounds__(W* Rows) void tiled_step(const void* __restrict__ src, void* __restrict__ dst,
+                                                      const Geometry g,
+                                                      const Physics<typename Storage<T>::Real> p, uint32_t tiles_x) {
+    __shared__ T tile[Q * W * H];
+    const int rx = static_cast<int>(threadIdx.x) % W, ry0 = static_cast<int>(threadIdx.x) / W;
+    const uint32_t bx = blockIdx.x % tiles_x, by = blockIdx.x / tiles_x;
+    const int x0 = static_cast<int>(bx) * (W - 2 * K), y0 = static_cast<int>(by) * (H - 2 * K);
+    const int w = min(W, static_cast<int>(g.nx) - x0 + 2 * K), h = min(H, static_cast<int>(g.ny) - y0 + 2 * K);
+    int xx = x0 + rx - K;  // beyond w: not used
+    if (xx < 0) xx += static_cast<int>(g.nx);
+    if (xx >= static_cast<int>(g.nx)) xx -= static_cast<int>(g.nx);
+    const uint32_t x = static_cast<uint32_t>(xx);
+    if constexpr (Bounded) {
+        // A tile whose cells are all plain fluid with plain-fluid neighbours takes the periodic path.
+        int marked = 0;
+        if (rx < w && (rx == 0 || rx == w - 1 || (x & 63U) == 0U))  // one lane of every segment touched
+            for (int ry = ry0; ry < h; ry += Rows) {
+                int yy = y0 + ry - K;
+                if (yy < 0) yy += static_cast<int>(g.ny);
+                if (yy >= static_cast<int>(g.ny)) yy -= static_cast<int>(g.ny);
+                marked |= static_cast<int>(p.segments[static_cast<uint32_t>(yy) * p.seg_x + (x >> 6)] & kSpanBits);
+            }
+        if (__syncthreads_or(marked) != 0) {
+            advance_tile<T, true, Forced, K, W, H, Rows>(src, dst, g, p, tile, rx, ry0, x, y0 - K, w, h);
+            return;
+        }
+    }
+    advance_tile<T, false, Forced, K, W, H, Rows>(src, dst, g, p, tile, rx, ry0, x, y0 - K, w, h);
+}
+
+constexpr uint32_t kHalo = 4;  // the largest K
+
+// Two tiles.  64 x 34 slots (FP32: 77 KiB of LDS, two blocks a CU; one wavefront a row) recompute 17 %
+// of the cells at K = 4 and are bound by the vector units: 4096^2 cavity FP32 134 us a step against 201
+// single (periodic 127 against 201, FP16S 91 against 115), 1400^2 15.1 against 26.2.  26 rows measure
+// 137-142, 42 rows 152, 8 rows of threads instead of 16 139.  Below about 200 000 cells they are too
+// few to fill the chip, and the launch and the chain of levels count: 32 x 16 slots, one cell a thread
+// (256^2 FP32: 2.0 us a step against 4.2 single and 2.9 in the large tile; 400^2: 2.8 against 5.5 and
+// 3.0; 600^2: 4.6 against 9.4 and 3.6).
+constexpr uint32_t kLargeTileCells = 200000U;
+
+template <class T, bool Bounded, bool Forced, int K> void launch(const LaunchState& st, const void* src, void* dst) {
+    using Real = typename Storage<T>::Real;
+    const auto go = [&](auto kernel, uint32_t w, uint32_t h, uint32_t threads) {
+        const uint32_t tx = (st.geo.nx + w - 2U * K - 1U) / (w - 2U * K), ty = (st.geo.ny + h - 2U * K - 1U) / (h - 2U * K);
+        hipLaunchKernelGGL(kernel, dim3(tx * ty), dim3(threads), 0, st.stream, src, dst, st.geo,
+                           *static_cast<const Physics<Real>*>(st.physics), tx);
+    };
+    if (st.cells >= kLargeTileCells) go(tiled_step<T, Bounded, Forced, K, 64, 34, 16>, 64U, 34U, 1024U);
+    else go(tiled_step<T, Bounded, Forced, K, 32, 16, 14>, 32U, 16U, 448U);
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess)
+        throw std::runtime_error(std::string("tiled_step launch: ") + hipGetErrorString(e));
+}
+
+template <class T> void steps(const LaunchState& st, int k, bool bounded, bool forced, const void* src, void* dst) {
+    const auto with = [&](auto B, auto F) {
+        constexpr bool b = decltype(B)::value, f = decltype(F)::value;
+        if (k == 4) launch<T, b, f, 4>(st, src, dst);
+        else if (k == 2) launch<T, b, f, 2>(st, src, dst);
+        else throw std::invalid_argument("tiled_steps takes 2 or 4 steps");
+    };
+    if (bounded) forced ? with(std::true_type{}, std::true_type{}) : with(std::true_type{}, std::false_type{});
+    else forced ? with(std::false_type{}, std::true_type{}) : with(std::false_type{}, std::false_type{});
+}
+
+}  // namespace
+
+bool tiled_supported(int q, int storage, size_t nx, size_t ny) {
+    // The coordinates wrap once, so the lattice is at least as large as the halo; FP64 stays with the
+    // single step (its tile would be half as large).
+    return q == 9 && (storage == 0 || storage == 1 || storage == 3) && nx >= 2 * kHalo && ny >= 2 * kHalo;
+}
+
+void tiled_steps(int storage, const LaunchState& st, int k, bool bounded, bool forced, const void* src, void* dst) {
+    switch (storage) {
+    case 0: return steps<float>(st, k, bounded, forced, src, dst);
+    case 1: return steps<_Float16>(st, k, bounded, forced, src, dst);
+    case 3: return steps<F32Dev>(st, k, bounded, forced, src, dst);
+    default: throw std::invalid_argument("tiled_steps: storage must be FP32, FP16S or FP32S");
+    }
+}
+
+}  // namespace cfd_hip
