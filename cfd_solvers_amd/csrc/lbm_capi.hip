@@ -81,9 +81,12 @@ template <class T> struct DeviceBuffer {
 
 namespace {
 // Zero fill by a kernel rather than hipMemsetAsync, so that callers may capture it in a graph.
+// `p` is the start of an allocation (16-byte aligned): four words a thread (85 MB: 13 us, 23 with one).
 __global__ void __launch_bounds__(256) zero_words_kernel(uint32_t* p, uint64_t words) {
-    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < words) p[i] = 0U;
+    const uint64_t i = 4U * (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x);
+    if (i + 4U <= words) *reinterpret_cast<uint4*>(p + i) = uint4{0U, 0U, 0U, 0U};
+    else
+        for (uint64_t k = i; k < words; ++k) p[k] = 0U;
 }
 }  // namespace
 
@@ -317,7 +320,9 @@ struct cfd_lbm_solver {
     // gives each XCD one run of rows: its L2 then holds the lines that neighbouring rows share, and a
     // line written in parts is completed in one L2 (D3Q27 56^3: 7.4 us a step against 10.8 round-robin;
     // D3Q19 FP16S 150^3: 42 against 59; D3Q19 FP32 128^3 cavity: 49.5 against 54.6; D2Q9 600^2: 6.4
-    // against 9.4).  On larger lattices long runs cost HBM locality (512^2 x 256 FP16S: 1099 us in one
+    // against 9.4).  Rows of whole lines in a lattice that the L2s hold together gain nothing from it
+    // (64^3 FP32, 100 steps and fields: 763 us against 748 round-robin; FP16S 615 against 583).  On larger
+    // lattices long runs cost HBM locality (512^2 x 256 FP16S: 1099 us in one
     // run each, 1005 round-robin), and only rows that are not whole 128-byte lines share lines: runs of
     // 8 tiles there (D3Q27 200^3: 324 us against 364; 190 x 150 x 141 FP32S: 111 against 122), single
     // tiles elsewhere (4096^2 D2Q9: 203 us against 211 in runs of 8).
@@ -328,8 +333,11 @@ struct cfd_lbm_solver {
             return g <= 0 ? 0U : (g == 1 ? run : static_cast<uint32_t>(std::min<long>(g, run)));
         }
         if (step_geo.tiles > (1U << 22)) return 0U;  // the padding to whole runs stays far below the grid's limit
-        if (pop_elems * elem <= (uint64_t{256} << 20)) return run;
-        return nx * elem % 128U != 0 ? std::min(8U, run) : 0U;
+        const bool whole_lines = nx * elem % 128U == 0;
+        const uint64_t bytes = pop_elems * elem;
+        if (whole_lines && bytes <= (uint64_t{32} << 20)) return 0U;
+        if (bytes <= (uint64_t{256} << 20)) return run;
+        return whole_lines ? 0U : std::min(8U, run);
     }
 
     void use_device() const { hip_check(hipSetDevice(device), "hipSetDevice"); }
@@ -1232,7 +1240,7 @@ struct cfd_lbm_solver {
     }
 
     void zero_words(unsigned char* p, uint64_t words) {
-        const uint64_t blocks = (words + 255) / 256;
+        const uint64_t blocks = (words + 1023) / 1024;
         if (blocks > 0x7FFFFFFFull) throw std::invalid_argument("buffer too large to clear");
         if (blocks) zero_words_kernel<<<static_cast<uint32_t>(blocks), 256, 0, stream>>>(reinterpret_cast<uint32_t*>(p), words);
         hip_check(hipGetLastError(), "zero_words");
