@@ -950,7 +950,8 @@ struct cfd_lbm_solver {
     // then the discrete adjoint back to the current state.  Checkpointing:
     //  * every > 0: two-level -- a snapshot every `every` steps on the way forward, and per segment
     //    an out-of-place recomputation of its states into replay buffers before the transposed
-    //    steps run through them (each step recomputed once; memory steps/every + every - 1 states);
+    //    steps run through them (each step but the last segment's recomputed once; memory
+    //    steps/every + every - 1 states);
     //  * every == 0: binomial -- `snapshots` state buffers (0: as many as fit, keeping 1/16 of the
     //    free memory in reserve) plus the start state, optimal recomputation (checkpoint_schedule.hpp).
     // grad_on_device: grad_gamma_out is device memory (cells doubles) and receives the gradient
@@ -1035,7 +1036,12 @@ struct cfd_lbm_solver {
         std::vector<std::pair<uint64_t, void*>> shots;
         std::vector<void*> free_list;
         if (every > 0) {
-            for (uint64_t c = 0; c * every < steps; ++c) shots.emplace_back(c * every, pool[c]);
+            // A snapshot every `every` steps, and every state of the last segment: the reverse phase
+            // starts there, so the forward sweep leaves them where a recomputation would put them.
+            const uint64_t segments = (steps + every - 1) / every;
+            for (uint64_t c = 0; c < segments; ++c) shots.emplace_back(c * every, pool[c]);
+            for (uint64_t k = (segments - 1) * every + 1; k < steps; ++k)
+                shots.emplace_back(k, pool[k - (segments - 1) * every - 1 + segments]);
         } else {
             shots.emplace_back(0, pool[0]);
             for (size_t k = 1; k < buffers; ++k) free_list.push_back(pool[k]);
@@ -1084,14 +1090,14 @@ struct cfd_lbm_solver {
         args.add_objective = 0;
         adj->seed(st, par(steps), b, lam, args);
         if (every > 0) {
-            const uint64_t segments = shots.size();
+            const uint64_t segments = (steps + every - 1) / every;
             for (uint64_t c = segments; c-- > 0;) {
                 const uint64_t s0 = c * every, e = std::min(steps, s0 + every);
                 std::vector<const void*> states(e - s0);
                 states[0] = shots[c].second;
                 for (uint64_t k = 1; k < e - s0; ++k) {
                     void* dst = pool[segments + k - 1];
-                    advance(states[k - 1], dst, s0 + k - 1, s0 + k);
+                    if (c + 1 < segments) advance(states[k - 1], dst, s0 + k - 1, s0 + k);
                     states[k] = dst;
                 }
                 for (uint64_t k = e - s0; k-- > 0;) transposed(s0 + k, states[k]);

@@ -192,8 +192,8 @@ CFD_LBM_API int cfd_lbm_objective_run(cfd_lbm_solver* s, int objective_kind, uin
                                       int x_out, double* objective, char* error, size_t error_capacity);
 /* Discrete adjoint (no reference counterpart: the reference has no adjoint).  Runs `steps` steps
  * from the current state, J = mean of the pressure drop over the last `window` states, then the
- * transposed steps back with a snapshot every `checkpoint_every` steps (two-level: each step is
- * recomputed once; memory ceil(steps/every) + every - 1 states); returns J, dJ/dgamma per cell
+ * transposed steps back with a snapshot every `checkpoint_every` steps (two-level: each step but
+ * the last segment's is recomputed once; memory ceil(steps/every) + every - 1 states); returns J, dJ/dgamma per cell
  * (cells doubles, may be NULL) and dJ/du_peak.  The state is left at time + steps.  Unforced
  * lattices with walls at rest, PBB, inlet and outlet; any storage (FP16: the adjoint of the FP32
  * collision at the stored states, lambda in FP32). */

@@ -64,3 +64,13 @@ def test_device_gradient_of_the_two_level_plan(hip, dev):
     assert np.array_equal(dev.download(grad, s.shape, np.float64), want[1])
     with pytest.raises(RuntimeError, match="aligned"):
         s.adjoint_run_device(12, 4, 4, 0)
+
+
+@pytest.mark.parametrize("every", [1, 4, 5, 11, 12, 40])
+def test_two_level_plans_agree(hip, every):
+    """The last segment's states are those of the forward sweep, the others' are recomputed: whatever
+    the interval (one state a segment, a short last segment, one segment), the binomial plan's J and
+    gradients, bit for bit."""
+    report("two_level_plan", every=every)
+    s = _solver(hip, (19, 14, 12), "fp32")
+    assert _same(_run(s, every, 0), _run(s, 0, 3))
