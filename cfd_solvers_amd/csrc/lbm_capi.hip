@@ -209,7 +209,7 @@ struct cfd_lbm_solver {
         step_geo = geo;
         const uint32_t width = step_width();
         tile_geometry(step_geo, width, width < 256U ? 256U / width : 1U);
-        step_geo.xcd_group = xcd_group();
+        step_geo.xcd_group = xcd_group(true);
         // Resident wavefronts per SIMD of the step kernel, bounded and periodic, capped by reserving
         // LDS per block (160 KiB per CU; a 256-thread block puts one wave on each of the 4 SIMDs).
         // Measured on MI355X:
@@ -325,8 +325,11 @@ struct cfd_lbm_solver {
     // lattices long runs cost HBM locality (512^2 x 256 FP16S: 1099 us in one
     // run each, 1005 round-robin), and only rows that are not whole 128-byte lines share lines: runs of
     // 8 tiles there (D3Q27 200^3: 324 us against 364; 190 x 150 x 141 FP32S: 111 against 122), single
-    // tiles elsewhere (4096^2 D2Q9: 203 us against 211 in runs of 8).
-    uint32_t xcd_group() const {
+    // tiles elsewhere (4096^2 D2Q9: 203 us against 211 in runs of 8).  An adjoint run goes through many
+    // states and lambda, so the caches hold none of them however small one is: in_place = false there
+    // (drag gradient of 60 steps, 145^3 FP32: 25.3 ms in runs of 8, 27.0 in one run each; 96^3: 7.05
+    // round-robin, 7.43).
+    uint32_t xcd_group(bool in_place) const {
         const uint32_t run = (step_geo.tiles + 7U) / 8U;
         if (const char* v = std::getenv("CFD_LBM_XCD_REMAP")) {  // tuning: 0 round-robin, 1 one run each, n: n tiles
             const long g = std::atol(v);
@@ -336,7 +339,7 @@ struct cfd_lbm_solver {
         const bool whole_lines = nx * elem % 128U == 0;
         const uint64_t bytes = pop_elems * elem;
         if (whole_lines && bytes <= (uint64_t{32} << 20)) return 0U;
-        if (bytes <= (uint64_t{256} << 20)) return run;
+        if (in_place && bytes <= (uint64_t{256} << 20)) return run;
         return whole_lines ? 0U : std::min(8U, run);
     }
 
@@ -1013,7 +1016,8 @@ struct cfd_lbm_solver {
         double* const peak_sums = acc + 1;
         args.grad_gamma = grad_on_device ? grad_gamma_out : reinterpret_cast<double*>(base + gg_at);
         args.grad_peak = reinterpret_cast<double*>(base + gp_at);
-        const LaunchState st = state();
+        LaunchState st = state();
+        st.step_geo.xcd_group = xcd_group(false);
         adj->zero(st, args.grad_gamma, cells);
         adj->zero(st, args.grad_peak, cells);
         adj->zero(st, acc, 1);
