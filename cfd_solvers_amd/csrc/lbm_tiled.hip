@@ -24,9 +24,10 @@ namespace cfd_hip {
 namespace {
 
 constexpr int Q = 9;
+constexpr int W = 64;  // slots of a tile row
 
 // Populations of the cell at LDS slot `c` (Odd: parity of the step), and back.
-template <class T, bool Odd, bool Bounded, int W, int P>
+template <class T, bool Odd, bool Bounded, int P>
 __device__ __forceinline__ void load_tile(const T* t, int c, uint32_t desc, typename Storage<T>::Real (&f)[Q]) {
     using L = Lattice<Q>;
     using S = Storage<T>;
@@ -44,7 +45,7 @@ __device__ __forceinline__ void load_tile(const T* t, int c, uint32_t desc, type
         }
     });
 }
-template <class T, bool Odd, int W, int P>
+template <class T, bool Odd, int P>
 __device__ __forceinline__ void store_tile(T* t, int c, const typename Storage<T>::Real (&f)[Q]) {
     using L = Lattice<Q>;
     using S = Storage<T>;
@@ -58,8 +59,8 @@ __device__ __forceinline__ void store_tile(T* t, int c, const typename Storage<T
 }
 
 // All K levels of one tile: W x H slots in LDS, the thread's column rx, rows ry0, ry0 + Rows, ...;
-// `w` x `h` of them lie within the lattice's last cell and its halo.
-template <class T, bool Bounded, bool Forced, int K, int W, int H, int Rows>
+// `w` x `h` of them are used: the interior, which ends with the lattice, and its halo.
+template <class T, bool Bounded, bool Forced, int K, int H, int Rows>
 __device__ __forceinline__ void advance_tile(const void* src, void* dst, const Geometry& g,
                                              const Physics<typename Storage<T>::Real>& p, T* t, int rx, int ry0,
                                              uint32_t x, int y_first, int w, int h) {
@@ -86,7 +87,7 @@ __device__ __forceinline__ void advance_tile(const void* src, void* dst, const G
                     PairSlots<Q> slots;
                     load_cell<Q, T, Odd, Bounded>(src, g, desc, neighbourhood(g, x, y, 0U), f, slots);
                 } else {
-                    load_tile<T, Odd, Bounded, W, P>(t, c, desc, f);
+                    load_tile<T, Odd, Bounded, P>(t, c, desc, f);
                 }
                 [[maybe_unused]] Real fin[Q];
                 if constexpr (Bounded && s == K)
@@ -95,7 +96,7 @@ __device__ __forceinline__ void advance_tile(const void* src, void* dst, const G
                                                        static_cast<uint8_t>(type), n, y, 0U, f);
                 if constexpr (s < K) {
                     if constexpr (Bounded) moving_wall_terms<Q, S>(p, desc, n, rho, f);
-                    store_tile<T, Odd, W, P>(t, c, f);
+                    store_tile<T, Odd, P>(t, c, f);
                 } else {
                     const Neighbourhood nb = neighbourhood(g, x, y, 0U);
                     PairSlots<Q> slots;
@@ -123,15 +124,16 @@ __device__ __forceinline__ void advance_tile(const void* src, void* dst, const G
     });
 }
 
-template <class T, bool Bounded, bool Forced, int K, int W, int H, int Rows>
+template <class T, bool Bounded, bool Forced, int K, int H, int Rows>
 __global__ __launch_bounds__(W* Rows) void tiled_step(const void* __restrict__ src, void* __restrict__ dst,
                                                       const Geometry g,
-                                                      const Physics<typename Storage<T>::Real> p, uint32_t tiles_x) {
+                                                      const Physics<typename Storage<T>::Real> p, uint32_t tiles_x,
+                                                      uint32_t rows) {
     __shared__ T tile[Q * W * H];
     const int rx = static_cast<int>(threadIdx.x) % W, ry0 = static_cast<int>(threadIdx.x) / W;
     const uint32_t bx = blockIdx.x % tiles_x, by = blockIdx.x / tiles_x;
-    const int x0 = static_cast<int>(bx) * (W - 2 * K), y0 = static_cast<int>(by) * (H - 2 * K);
-    const int w = min(W, static_cast<int>(g.nx) - x0 + 2 * K), h = min(H, static_cast<int>(g.ny) - y0 + 2 * K);
+    const int x0 = static_cast<int>(bx) * (W - 2 * K), y0 = static_cast<int>(by * rows);
+    const int w = min(W, static_cast<int>(g.nx) - x0 + 2 * K), h = min(static_cast<int>(rows), static_cast<int>(g.ny) - y0) + 2 * K;
     int xx = x0 + rx - K;  // beyond w: not used
     if (xx < 0) xx += static_cast<int>(g.nx);
     if (xx >= static_cast<int>(g.nx)) xx -= static_cast<int>(g.nx);
@@ -147,33 +149,53 @@ __global__ __launch_bounds__(W* Rows) void tiled_step(const void* __restrict__ s
                 marked |= static_cast<int>(p.segments[static_cast<uint32_t>(yy) * p.seg_x + (x >> 6)] & kSpanBits);
             }
         if (__syncthreads_or(marked) != 0) {
-            advance_tile<T, true, Forced, K, W, H, Rows>(src, dst, g, p, tile, rx, ry0, x, y0 - K, w, h);
+            advance_tile<T, true, Forced, K, H, Rows>(src, dst, g, p, tile, rx, ry0, x, y0 - K, w, h);
             return;
         }
     }
-    advance_tile<T, false, Forced, K, W, H, Rows>(src, dst, g, p, tile, rx, ry0, x, y0 - K, w, h);
+    advance_tile<T, false, Forced, K, H, Rows>(src, dst, g, p, tile, rx, ry0, x, y0 - K, w, h);
 }
 
 constexpr uint32_t kHalo = 4;  // the largest K
 
-// Two tiles.  64 x 34 slots (FP32: 77 KiB of LDS, two blocks a CU; one wavefront a row) recompute 17 %
-// of the cells at K = 4 and are bound by the vector units: 4096^2 cavity FP32 134 us a step against 201
-// single (periodic 127 against 201, FP16S 91 against 115), 1400^2 15.1 against 26.2.  26 rows measure
-// 137-142, 42 rows 152, 8 rows of threads instead of 16 139.  Below about 200 000 cells they are too
-// few to fill the chip, and the launch and the chain of levels count: 32 x 16 slots, one cell a thread
-// (256^2 FP32: 2.0 us a step against 4.2 single and 2.9 in the large tile; 400^2: 2.8 against 5.5 and
-// 3.0; 600^2: 4.6 against 9.4 and 3.6).
+// Two tiles, both 64 slots (one wavefront) wide.  34 rows (FP32: 77 KiB of LDS, two blocks a CU)
+// recompute 17 % of the cells at K = 4 and are bound by the vector units: 4096^2 cavity FP32 134 us a
+// step against 201 single (periodic 127 against 201, FP16S 91 against 115), 1400^2 15.1 against 26.2.
+// 26 rows measure 137-142, 42 rows 152, 8 rows of threads instead of 16 139.
+//
+// Below about 200 000 cells those tiles are too few to fill the chip, and the launch and the chain of
+// levels count: up to 16 rows, 12 of them at a time, and as many interior rows as make the fewest
+// wavefronts of the busiest CU (tile_rows).  256^2 FP32: 2.0 us a step against 4.2 single and 2.9 in
+// the large tile; 330^2: 2.2; 400^2: 2.6 against 5.5 and 3.0; 100 x 500: 1.9.  Tiles of 32 x 16 slots
+// measure 2.1, 2.4, 2.9 and 2.1; the large tile is ahead at 600^2 (3.6 against 4.6).
 constexpr uint32_t kLargeTileCells = 200000U;
+
+// Interior rows (2 to `most`) of tiles with `strips` columns: blocks are dealt to 256 CUs, and a block
+// issues K rows + K (K - 1) wavefronts over its levels (rows + 2 (K - s) at level s).
+uint32_t tile_rows(uint32_t strips, uint32_t ny, uint32_t k, uint32_t most) {
+    uint32_t best = most;
+    uint64_t least = ~uint64_t{0};
+    for (uint32_t rows = most; rows >= 2U; --rows) {
+        const uint64_t blocks = static_cast<uint64_t>(strips) * ((ny + rows - 1U) / rows);
+        const uint64_t waves = (blocks + 255U) / 256U * (k * rows + k * (k - 1U));
+        if (waves < least) {
+            least = waves;
+            best = rows;
+        }
+    }
+    return best;
+}
 
 template <class T, bool Bounded, bool Forced, int K> void launch(const LaunchState& st, const void* src, void* dst) {
     using Real = typename Storage<T>::Real;
-    const auto go = [&](auto kernel, uint32_t w, uint32_t h, uint32_t threads) {
-        const uint32_t tx = (st.geo.nx + w - 2U * K - 1U) / (w - 2U * K), ty = (st.geo.ny + h - 2U * K - 1U) / (h - 2U * K);
-        hipLaunchKernelGGL(kernel, dim3(tx * ty), dim3(threads), 0, st.stream, src, dst, st.geo,
-                           *static_cast<const Physics<Real>*>(st.physics), tx);
+    constexpr uint32_t kInner = 64U - 2U * K;
+    const uint32_t tx = (st.geo.nx + kInner - 1U) / kInner;
+    const auto go = [&](auto kernel, uint32_t rows, uint32_t threads) {
+        hipLaunchKernelGGL(kernel, dim3(tx * ((st.geo.ny + rows - 1U) / rows)), dim3(threads), 0, st.stream, src, dst,
+                           st.geo, *static_cast<const Physics<Real>*>(st.physics), tx, rows);
     };
-    if (st.cells >= kLargeTileCells) go(tiled_step<T, Bounded, Forced, K, 64, 34, 16>, 64U, 34U, 1024U);
-    else go(tiled_step<T, Bounded, Forced, K, 32, 16, 14>, 32U, 16U, 448U);
+    if (st.cells >= kLargeTileCells) go(tiled_step<T, Bounded, Forced, K, 34, 16>, 34U - 2U * K, 1024U);
+    else go(tiled_step<T, Bounded, Forced, K, 16, 12>, tile_rows(tx, st.geo.ny, K, 16U - 2U * K), 768U);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess)
         throw std::runtime_error(std::string("tiled_step launch: ") + hipGetErrorString(e));
 }

@@ -9,8 +9,9 @@ from conftest import report
 
 pytestmark = pytest.mark.gpu
 
-# The small tile's interior is 24 x 8 (2 steps: 28 x 12), the large one's 56 x 26 (60 x 30).
-SMALL = [(8, 8), (24, 8), (25, 17), (57, 9), (131, 40)]
+# A tile's interior is 56 wide (2 steps: 60); the small one has 2 to 8 rows (2 steps: to 12) by the
+# lattice's size, the large one 26 (30).
+SMALL = [(8, 8), (24, 8), (25, 17), (57, 9), (131, 40), (2300, 15), (171, 700)]
 LARGE = [(448, 520), (449, 469), (9, 22300)]
 
 
