@@ -3,9 +3,10 @@
 // hipMalloc and hipFree of a large block cost far more than the kernels that use it: mapping and
 // clearing run at about 40 GB/s, so the 16.8 GB of checkpoint states of a 200-step two-level adjoint
 // on 128^3 took 410 ms of a 457 ms call.  A call that needs such a block for its own duration takes it
-// from WorkspacePool, which keeps the blocks of finished calls for the next one, of whichever solver:
-// at most kKeptFraction of the device's memory, given back when the last solver goes and before any
-// allocation of this library fails.
+// from WorkspacePool (Workspace), which keeps the blocks of finished calls for the next one, of
+// whichever solver; a block that one object wants at every call it holds itself (HeldBlock).  Neither
+// holds a state between calls.  Idle and held blocks are each bounded to 1 / kKeptFraction of the
+// device's memory, and both are given back before any allocation of this library fails.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,6 +18,8 @@
 #include <vector>
 
 namespace cfd_hip {
+
+class HeldBlock;
 
 class WorkspacePool {
   public:
@@ -31,6 +34,8 @@ class WorkspacePool {
 
     // A block of at least `bytes` on the current device, for the caller alone until put().
     unsigned char* take(size_t bytes, size_t* got);
+    // The same from the idle blocks only; null if none fits.
+    unsigned char* take_idle(size_t bytes, size_t* got);
     // Ends the use of a block of the current device; no work that uses it is pending.
     void put(unsigned char* ptr, size_t bytes, bool keep);
     // Bytes of the idle blocks on the current device.
@@ -38,11 +43,9 @@ class WorkspacePool {
         const std::lock_guard<std::mutex> lock(mutex_);
         return idle_bytes_locked(current_device());
     }
-    // Gives back the idle blocks of the current device; false if there were none.
-    bool trim() {
-        const std::lock_guard<std::mutex> lock(mutex_);
-        return trim_locked(current_device(), 0);
-    }
+    // Gives back the current device's idle blocks and the held ones that no call is using; false if
+    // there were none.
+    bool trim();
     // Users (solvers) alive; the last one to leave gives back every idle block.
     void enter() {
         const std::lock_guard<std::mutex> lock(mutex_);
@@ -57,6 +60,7 @@ class WorkspacePool {
     }
 
   private:
+    friend class HeldBlock;
     struct Block {
         unsigned char* ptr;
         size_t bytes;
@@ -88,10 +92,72 @@ class WorkspacePool {
         return any;
     }
 
+    static size_t bound() {
+        size_t total = 0;
+        return hipDeviceTotalMem(&total, current_device()) == hipSuccess ? total / kKeptFraction : 0;
+    }
+
     std::mutex mutex_;
     std::vector<Block> idle_;  // oldest first
+    std::vector<HeldBlock*> held_;
     size_t users_ = 0;
 };
+
+// A block that its owner keeps from call to call: take() before its use, done() once the work on it
+// has been launched (on one stream, which the owner waits for before it goes).  Between the two calls
+// a full device may take it away, after waiting for that work.
+class HeldBlock {
+  public:
+    HeldBlock() = default;
+    HeldBlock(const HeldBlock&) = delete;
+    HeldBlock& operator=(const HeldBlock&) = delete;
+    ~HeldBlock() {
+        WorkspacePool& pool = WorkspacePool::instance();
+        {
+            const std::lock_guard<std::mutex> lock(pool.mutex_);
+            forget(pool);
+        }
+        if (ptr_) pool.put(ptr_, bytes_, true);
+    }
+    // The block, of `bytes` bytes at every call; null if there is no room for it.
+    unsigned char* take(size_t bytes);
+    void done() {
+        const std::lock_guard<std::mutex> lock(WorkspacePool::instance().mutex_);
+        busy_ = false;
+    }
+    size_t bytes() const { return bytes_; }
+
+  private:
+    friend class WorkspacePool;
+    void forget(WorkspacePool& pool) {  // with the pool locked
+        for (size_t k = 0; k < pool.held_.size(); ++k)
+            if (pool.held_[k] == this) {
+                pool.held_.erase(pool.held_.begin() + static_cast<std::ptrdiff_t>(k));
+                return;
+            }
+    }
+    unsigned char* ptr_ = nullptr;
+    size_t bytes_ = 0;
+    int device_ = 0;
+    bool busy_ = false;
+    bool refused_ = false;  // the device was full once: not tried again
+};
+
+inline bool WorkspacePool::trim() {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    const int device = current_device();
+    bool any = trim_locked(device, 0);
+    for (size_t k = held_.size(); k-- > 0;) {
+        HeldBlock* const h = held_[k];
+        if (h->busy_ || h->device_ != device) continue;
+        (void)hipFree(h->ptr_);  // waits for the device, and with it for the block's last use
+        h->ptr_ = nullptr;
+        h->bytes_ = 0;
+        held_.erase(held_.begin() + static_cast<std::ptrdiff_t>(k));
+        any = true;
+    }
+    return any;
+}
 
 // hipMalloc on the current device; when that finds the device full, once more after the idle
 // workspaces have been given back.
@@ -102,23 +168,24 @@ inline hipError_t device_malloc(void** p, size_t bytes) {
     return hipMalloc(p, bytes);
 }
 
+inline unsigned char* WorkspacePool::take_idle(size_t bytes, size_t* got) {
+    // The smallest idle block that holds the request, unless it would waste more than half of it.
+    const std::lock_guard<std::mutex> lock(mutex_);
+    const int device = current_device();
+    size_t best = idle_.size();
+    for (size_t k = 0; k < idle_.size(); ++k)
+        if (idle_[k].device == device && idle_[k].bytes >= bytes && idle_[k].bytes / 2 <= bytes &&
+            (best == idle_.size() || idle_[k].bytes < idle_[best].bytes))
+            best = k;
+    if (best == idle_.size()) return nullptr;
+    unsigned char* const p = idle_[best].ptr;
+    *got = idle_[best].bytes;
+    idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(best));
+    return p;
+}
+
 inline unsigned char* WorkspacePool::take(size_t bytes, size_t* got) {
-    {
-        // The smallest idle block that holds the request, unless it would waste more than half of it.
-        const std::lock_guard<std::mutex> lock(mutex_);
-        const int device = current_device();
-        size_t best = idle_.size();
-        for (size_t k = 0; k < idle_.size(); ++k)
-            if (idle_[k].device == device && idle_[k].bytes >= bytes && idle_[k].bytes / 2 <= bytes &&
-                (best == idle_.size() || idle_[k].bytes < idle_[best].bytes))
-                best = k;
-        if (best < idle_.size()) {
-            unsigned char* const p = idle_[best].ptr;
-            *got = idle_[best].bytes;
-            idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(best));
-            return p;
-        }
-    }
+    if (unsigned char* const p = take_idle(bytes, got)) return p;
     void* p = nullptr;
     if (const hipError_t e = device_malloc(&p, bytes); e != hipSuccess)
         throw std::runtime_error(std::string("hipMalloc: ") + hipGetErrorString(e));
@@ -128,17 +195,57 @@ inline unsigned char* WorkspacePool::take(size_t bytes, size_t* got) {
 
 inline void WorkspacePool::put(unsigned char* ptr, size_t bytes, bool keep) {
     const std::lock_guard<std::mutex> lock(mutex_);
-    size_t free_b = 0, total = 0;
-    if (keep && users_ > 0 && hipMemGetInfo(&free_b, &total) == hipSuccess && bytes <= total / kKeptFraction) {
+    if (const size_t most = bound(); keep && users_ > 0 && bytes <= most) {
         const int device = current_device();
         try {
-            trim_locked(device, total / kKeptFraction - bytes);
+            trim_locked(device, most - bytes);
             idle_.push_back(Block{ptr, bytes, device});
             return;
         } catch (...) {  // no host memory for the list: give the block back
         }
     }
     (void)hipFree(ptr);
+}
+
+inline unsigned char* HeldBlock::take(size_t bytes) {
+    WorkspacePool& pool = WorkspacePool::instance();
+    {
+        const std::lock_guard<std::mutex> lock(pool.mutex_);
+        if (ptr_) {
+            busy_ = true;
+            return ptr_;
+        }
+        if (refused_) return nullptr;
+        size_t sum = bytes;
+        const int device = WorkspacePool::current_device();
+        for (const HeldBlock* h : pool.held_)
+            if (h->device_ == device) sum += h->bytes_;
+        if (sum > WorkspacePool::bound()) return nullptr;
+    }
+    size_t got = 0;
+    unsigned char* p = pool.take_idle(bytes, &got);
+    if (!p) {  // a plain hipMalloc: what the caller can do without takes no block from another owner
+        void* fresh = nullptr;
+        if (hipMalloc(&fresh, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            refused_ = true;
+            return nullptr;
+        }
+        p = static_cast<unsigned char*>(fresh);
+        got = bytes;
+    }
+    const std::lock_guard<std::mutex> lock(pool.mutex_);
+    try {
+        pool.held_.push_back(this);
+    } catch (...) {  // no host memory for the list
+        (void)hipFree(p);
+        return nullptr;
+    }
+    ptr_ = p;
+    bytes_ = got;
+    device_ = WorkspacePool::current_device();
+    busy_ = true;
+    return ptr_;
 }
 
 // One block of the pool for the duration of a scope.  On the way out of a failed call the block is

@@ -128,9 +128,7 @@ struct cfd_lbm_solver {
     uint64_t last_forward_steps = 0;
     // The second lattice of the several-steps-per-launch kernels, taken at the first call that uses
     // them and held until the solver goes; the state is in `f` between calls.
-    unsigned char* second = nullptr;
-    size_t second_bytes = 0;
-    bool second_refused = false;
+    cfd_hip::HeldBlock second;
     mutable TransferStats stats;
     // Host copy of the Physics<Real> passed by value to every launch.
     alignas(16) unsigned char physics[sizeof(Physics<double>)] = {};
@@ -273,7 +271,6 @@ struct cfd_lbm_solver {
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
         }
-        if (second) cfd_hip::WorkspacePool::instance().put(second, second_bytes, true);
         cfd_hip::WorkspacePool::instance().leave();
     }
 
@@ -1256,25 +1253,14 @@ struct cfd_lbm_solver {
         hip_check(hipGetLastError(), "zero_words");
     }
 
-    // Whether `count` steps may run several to a launch (lbm_tiled.hip): an unporous D2Q9 lattice whose
-    // second copy is within the workspace bound, outside of stream capture (a graph is replayed on
-    // `f` alone, and it must not hold an allocation).
-    bool several_per_launch(uint64_t count) {
-        if (count < 4U || gamma || second_refused || !cfd_hip::tiled_supported(q, storage, nx, ny)) return false;
+    // The second lattice if `count` steps may run several to a launch (lbm_tiled.hip): an unporous D2Q9
+    // lattice whose second copy is within the workspace bound, outside of stream capture (a graph is
+    // replayed on `f` alone, and it must not hold an allocation).  Null: single steps.
+    unsigned char* second_lattice(uint64_t count) {
+        if (count < 4U || gamma || !cfd_hip::tiled_supported(q, storage, nx, ny)) return nullptr;
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
-        if (second) return true;
-        size_t free_b = 0, total = 0;
-        hip_check(hipMemGetInfo(&free_b, &total), "hipMemGetInfo");
-        second_refused = f.bytes > total / cfd_hip::WorkspacePool::kKeptFraction;
-        if (second_refused) return false;
-        try {
-            second = cfd_hip::WorkspacePool::instance().take(f.bytes, &second_bytes);
-        } catch (const std::runtime_error&) {  // no room: the single step needs none
-            (void)hipGetLastError();
-            second_refused = true;
-        }
-        return second != nullptr;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
+        return second.take(f.bytes);
     }
 
     void step(uint64_t count) {
@@ -1287,13 +1273,17 @@ struct cfd_lbm_solver {
             ++t;
             --count;
         };
-        if (several_per_launch(count - (odd() && count > 0 ? 1U : 0U))) {
+        if (unsigned char* const other = second_lattice(count - (odd() && count > 0 ? 1U : 0U))) {
+            struct Done {
+                cfd_hip::HeldBlock& block;
+                ~Done() { block.done(); }
+            } done{second};
             if (odd()) single();  // the tiled kernels start at even parity
             // Pairs of launches, f to the second lattice and back.
             for (int k = 4; k >= 2; k -= 2)
                 for (; count >= 2U * static_cast<uint64_t>(k); count -= 2U * static_cast<uint64_t>(k)) {
-                    cfd_hip::tiled_steps(storage, st, k, b, forced, f.ptr, second);
-                    cfd_hip::tiled_steps(storage, st, k, b, forced, second, f.ptr);
+                    cfd_hip::tiled_steps(storage, st, k, b, forced, f.ptr, other);
+                    cfd_hip::tiled_steps(storage, st, k, b, forced, other, f.ptr);
                     t += 2U * static_cast<uint64_t>(k);
                 }
         }
@@ -1302,7 +1292,7 @@ struct cfd_lbm_solver {
 
     float step_timed(uint64_t count) {
         use_device();
-        (void)several_per_launch(count);  // its allocation is not part of the steps
+        if (second_lattice(count)) second.done();  // its allocation is not part of the steps
         TimingEvent e0, e1;
         float ms = 0.0F;
         hip_check(hipEventRecord(e0.e, stream), "hipEventRecord");
@@ -1397,7 +1387,7 @@ struct cfd_lbm_solver {
     size_t population_bytes() const { return static_cast<size_t>(q) * cells * elem; }
     size_t resident_bytes() const {
         return f.bytes + flags.bytes + links.bytes + link_vel.bytes + segments.bytes + solid_rho.bytes + gamma.bytes + lacc.bytes + macro.bytes + partial.bytes +
-               reduce_out.bytes + second_bytes;
+               reduce_out.bytes + second.bytes();
     }
 };
 
