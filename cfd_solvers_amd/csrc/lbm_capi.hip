@@ -313,18 +313,22 @@ struct cfd_lbm_solver {
         return 64U * best;
     }
 
-    // Consecutive tiles of one XCD in the step kernels.  A lattice that fits the 256 MiB Infinity Cache
-    // gives each XCD one run of rows: its L2 then holds the lines that neighbouring rows share, and a
-    // line written in parts is completed in one L2 (D3Q27 56^3: 7.4 us a step against 10.8 round-robin;
-    // D3Q19 FP16S 150^3: 42 against 59; D3Q19 FP32 128^3 cavity: 49.5 against 54.6; D2Q9 600^2: 6.4
-    // against 9.4).  Rows of whole lines in a lattice that the L2s hold together gain nothing from it
-    // (64^3 FP32, 100 steps and fields: 763 us against 748 round-robin; FP16S 615 against 583).  On larger
-    // lattices long runs cost HBM locality (512^2 x 256 FP16S: 1099 us in one
-    // run each, 1005 round-robin), and only rows that are not whole 128-byte lines share lines: runs of
-    // 8 tiles there (D3Q27 200^3: 324 us against 364; 190 x 150 x 141 FP32S: 111 against 122), single
-    // tiles elsewhere (4096^2 D2Q9: 203 us against 211 in runs of 8).  An adjoint run goes through many
-    // states and lambda, so the caches hold none of them however small one is: in_place = false there
-    // (drag gradient of 60 steps, 145^3 FP32: 25.3 ms in runs of 8, 27.0 in one run each; 96^3: 7.05
+    // Consecutive tiles of one XCD in the step kernels.  A small lattice gives each XCD one run of rows:
+    // its L2 then holds the lines that neighbouring rows share, and a line written in parts is completed
+    // in one L2 (D3Q27 56^3: 7.4 us a step against 10.8 round-robin; 61 x 112 x 83 FP16S cavity, 20 steps
+    // and fields: 255 us against 299).  Rows of whole lines in a lattice that the L2s hold together gain
+    // nothing from it (64^3 FP32, 100 steps and fields: 763 us against 748 round-robin; FP16S 615 against
+    // 583).  Up to the 256 MiB of the Infinity Cache, one run each is fastest for a lattice that has the
+    // cache to itself but slowest when other solvers' lattices pass through it at the same time; runs of
+    // 32 tiles gain in both (20 steps and fields, alone / three solvers at once, round-robin, 32, one
+    // run: FP32 150^2 x 148 1880 / 2240, 1577 / 2012, 1533 / 2029 us; 105 x 180^2 channel 2041 / 2274,
+    // 1962 / 2288, 2091 / 2380; FP16S 192 x 128^2 cavity 1108 / 954, 1015 / 948, 879 / 956).  On larger
+    // lattices long runs cost HBM locality (512^2 x 256 FP16S: 1099 us a step in one run each, 1005
+    // round-robin), and only rows that are not whole 128-byte lines share lines: runs of 8 tiles there
+    // (D3Q27 200^3: 324 us against 364; 190 x 150 x 141 FP32S: 111 against 122), single tiles elsewhere
+    // (4096^2 D2Q9: 203 us against 211 in runs of 8).  An adjoint run goes through many states and
+    // lambda, so the caches hold none of them however small one is: in_place = false there (drag
+    // gradient of 60 steps, 145^3 FP32: 25.3 ms in runs of 8, 27.0 in one run each; 96^3: 7.05
     // round-robin, 7.43).
     uint32_t xcd_group(bool in_place) const {
         const uint32_t run = (step_geo.tiles + 7U) / 8U;
@@ -336,7 +340,8 @@ struct cfd_lbm_solver {
         const bool whole_lines = nx * elem % 128U == 0;
         const uint64_t bytes = pop_elems * elem;
         if (whole_lines && bytes <= (uint64_t{32} << 20)) return 0U;
-        if (in_place && bytes <= (uint64_t{256} << 20)) return run;
+        if (in_place && bytes <= (uint64_t{64} << 20)) return run;
+        if (in_place && bytes <= (uint64_t{256} << 20)) return std::min(32U, run);
         return whole_lines ? 0U : std::min(8U, run);
     }
 
