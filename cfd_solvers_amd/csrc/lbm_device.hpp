@@ -515,21 +515,11 @@ __device__ __forceinline__ void fluid_moments(const Real (&f)[Q], Real& rp, Real
     if constexpr (Lattice<Q>::dims == 2) uz = Real(0);
 }
 
-// The local body acceleration of cell n, loaded ahead of its populations so that both are in flight.
-template <class Real> __device__ __forceinline__ void local_acceleration(const Physics<Real>& p, uint32_t n, Real (&a)[3]) {
-    a[0] = a[1] = a[2] = Real(0);
-    if (p.lax) {
-        a[0] = p.lax[n];
-        a[1] = p.lax[p.cells + n];
-        a[2] = p.lax[2U * p.cells + n];
-    }
-}
-
 // Macroscopic state a non-wall cell reports (esoteric_pull.hpp:180-209 for fluid cells).
 template <int Q, class S, class Real>
 __device__ __forceinline__ void cell_state(const Physics<Real>& p, const Geometry& g, uint8_t flag, uint32_t n,
-                                           uint32_t y, uint32_t z, const Real (&f)[Q], const Real (&local)[3],
-                                           Real& rho, Real& ux, Real& uy, Real& uz) {
+                                           uint32_t y, uint32_t z, const Real (&f)[Q], Real& rho, Real& ux, Real& uy,
+                                           Real& uz) {
     if (flag == kInlet) {
         const Real uin = inlet_velocity(p, g, y, z, Lattice<Q>::dims == 3);
         Real rp;
@@ -548,9 +538,9 @@ __device__ __forceinline__ void cell_state(const Physics<Real>& p, const Geometr
     fluid_moments<S, Q>(f, rp, rho, ux, uy, uz);
     Real ax = p.ax, ay = p.ay, az = p.az;
     if (p.lax) {
-        ax = ax + local[0];
-        ay = ay + local[1];
-        az = az + local[2];
+        ax = ax + p.lax[n];
+        ay = ay + p.lax[p.cells + n];
+        az = az + p.lax[2U * p.cells + n];
     }
     ux = ux + Real(0.5) * ax;
     uy = uy + Real(0.5) * ay;

@@ -385,12 +385,11 @@ __global__ __launch_bounds__(kStepThreads<typename Storage<T>::Real>) void macro
             return;
         }
     }
-    Real fin[Q], local[3];
+    Real fin[Q];
     PairSlots<Q> s;
-    local_acceleration(p, n, local);
     load_cell<Q, T, Odd, Bounded>(f, g, link_desc<Bounded>(p.links, n), h, fin, s);
     Real rho, ux, uy, uz;
-    cell_state<Q, Storage<T>>(p, g, flag, n, y, z, fin, local, rho, ux, uy, uz);
+    cell_state<Q, Storage<T>>(p, g, flag, n, y, z, fin, rho, ux, uy, uz);
     out[n] = rho;
     out[cells + n] = ux;
     out[2U * cells + n] = uy;
@@ -478,9 +477,8 @@ __global__ __launch_bounds__(256) void diagnostics_partial(const void* __restric
             // Shifted storage: the sum of deviations is rho - 1 (added in FP64).
             mass = Storage<T>::kShifted ? 1.0 + static_cast<double>(sum * static_cast<Real>(Storage<T>::kInvScale))
                                         : static_cast<double>(sum);
-            Real rho, ux, uy, uz, local[3];
-            local_acceleration(p, n, local);
-            cell_state<Q, Storage<T>>(p, g, flag, n, y, z, fin, local, rho, ux, uy, uz);
+            Real rho, ux, uy, uz;
+            cell_state<Q, Storage<T>>(p, g, flag, n, y, z, fin, rho, ux, uy, uz);
             ke = static_cast<double>(rho) * (static_cast<double>(ux) * ux + static_cast<double>(uy) * uy +
                                              static_cast<double>(uz) * uz);
             vmax = static_cast<double>(sqrt(ux * ux + uy * uy + uz * uz));

@@ -48,3 +48,14 @@ def test_no_kernel_uses_scratch_memory(kernels):
     assert sum("14stream_collideI" in n for n in kernels) == 3 * 5 * 8 and sum("10tiled_stepI" in n for n in kernels) == 48
     used = {n: k[".private_segment_fixed_size"] for n, k in kernels.items() if k[".private_segment_fixed_size"]}
     assert not used, f"{len(used)} kernels, {list(used.items())[:3]}"
+
+
+def test_field_kernels_keep_their_waves(kernels):
+    """macroscopic and diagnostics_partial run 8 waves a SIMD on periodic lattices (64 of 512 vector
+    registers a lane) and at least 7 (72) on bounded ones; the largest are the D3Q27 FP64 ones."""
+    for kernel in ("11macroscopicI", "19diagnostics_partialI"):
+        for bounded, most in (("Lb0E", 64), ("Lb1E", 72)):
+            used = {n: k[".vgpr_count"] for n, k in kernels.items()
+                    if kernel in n and n.split(kernel)[1].split("EEvPKv")[0].endswith(bounded)}
+            assert len(used) == 3 * 5 * 2
+            assert max(used.values()) <= most, max(used.items(), key=lambda i: i[1])
