@@ -103,6 +103,23 @@ class WorkspacePool {
     size_t users_ = 0;
 };
 
+// For its lifetime the calling thread may allocate although some stream, of whichever thread, is being
+// captured: hipMalloc records nothing, but under a capture in global mode (torch's default) it fails
+// and ends that capture.
+class AllocationDuringCapture {
+  public:
+    AllocationDuringCapture() { set_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+    ~AllocationDuringCapture() {
+        if (set_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    AllocationDuringCapture(const AllocationDuringCapture&) = delete;
+    AllocationDuringCapture& operator=(const AllocationDuringCapture&) = delete;
+
+  private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool set_ = false;
+};
+
 // A block that its owner keeps from call to call: take() before its use, done() once the work on it
 // has been launched (on one stream, which the owner waits for before it goes).  Between the two calls
 // a full device may take it away, after waiting for that work.
@@ -225,6 +242,7 @@ inline unsigned char* HeldBlock::take(size_t bytes) {
     size_t got = 0;
     unsigned char* p = pool.take_idle(bytes, &got);
     if (!p) {  // a plain hipMalloc: what the caller can do without takes no block from another owner
+        const AllocationDuringCapture permit;  // a caller that steps expects no allocation
         void* fresh = nullptr;
         if (hipMalloc(&fresh, bytes) != hipSuccess) {
             (void)hipGetLastError();

@@ -1,0 +1,85 @@
+// Scenarios of the workspace pool on the stand-in device: 1600 bytes, so 100 may stay idle and 100 held.
+#include "device_memory.hpp"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <optional>
+
+using cfd_hip::HeldBlock;
+using cfd_hip::Workspace;
+using cfd_hip::WorkspacePool;
+
+#define EXPECT(c)                                                            \
+    do {                                                                     \
+        if (!(c)) {                                                          \
+            std::fprintf(stderr, "line %d: %s does not hold\n", __LINE__, #c); \
+            std::exit(1);                                                    \
+        }                                                                    \
+    } while (0)
+
+namespace {
+
+WorkspacePool& pool = WorkspacePool::instance();
+
+// A block that a finished call leaves idle.
+unsigned char* leave_idle(size_t bytes) {
+    Workspace w(bytes);
+    w.finished();
+    return w.get();
+}
+
+void reuse() {
+    pool.enter();
+    unsigned char* const first = leave_idle(80);
+    EXPECT(pool.idle_bytes() == 80);
+    EXPECT(leave_idle(60) == first && stub::mallocs == 1);  // reused, and idle again
+    EXPECT(leave_idle(30) != first);                        // more than half of it would be wasted: a block of its own
+    EXPECT(pool.idle_bytes() == 30);                        // 110 is over the bound: the oldest goes
+    { Workspace failed(30); }                               // never finished: given back
+    EXPECT(pool.idle_bytes() == 0);
+    leave_idle(101);                                        // over the bound
+    EXPECT(pool.idle_bytes() == 0 && stub::used == 0);
+    leave_idle(50);
+    pool.leave();
+    EXPECT(stub::used == 0);
+}
+
+void full_device() {
+    pool.enter();
+    HeldBlock busy, rests;
+    EXPECT(busy.take(40) && rests.take(40));
+    rests.done();
+    leave_idle(90);
+    void* p = nullptr;
+    EXPECT(cfd_hip::device_malloc(&p, stub::capacity - 40) == hipSuccess);  // all but the block in use
+    EXPECT(pool.idle_bytes() == 0 && rests.bytes() == 0 && busy.bytes() == 40);
+    EXPECT(cfd_hip::device_malloc(&p, 1) == hipErrorOutOfMemory);
+    busy.done();
+    EXPECT(cfd_hip::device_malloc(&p, 40) == hipSuccess);
+    EXPECT(busy.bytes() == 0);
+    EXPECT(!rests.take(40));  // full: the caller does without
+    pool.leave();
+}
+
+void foreign_capture() {
+    pool.enter();
+    stub::capturing = true;
+    HeldBlock h;
+    EXPECT(h.take(40));
+    EXPECT(!stub::broken && stub::mode == hipStreamCaptureModeGlobal);
+    h.done();
+    pool.leave();
+}
+
+}  // namespace
+
+int main(int, char** argv) {
+    const struct {
+        const char* name;
+        void (*run)();
+    } all[] = {{"reuse", reuse}, {"full_device", full_device}, {"foreign_capture", foreign_capture}};
+    for (const auto& s : all)
+        if (std::strcmp(argv[1], s.name) == 0) return s.run(), 0;
+    return 2;
+}

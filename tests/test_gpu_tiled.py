@@ -2,6 +2,8 @@
 the raw slots (those left behind at walls included), populations and fields, over both tile sizes,
 lattices at the halo's width, at tile edges and beyond them, odd and even starts and counts, and
 every option the step has."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -88,3 +90,27 @@ def test_other_lattices_take_single_steps(hip, kind):
     before = g.resident_bytes()
     g.step(8)
     assert g.resident_bytes() == before
+
+
+def test_first_call_during_a_capture_of_another_stream(hip):
+    """The call that takes the second lattice neither ends a global-mode capture of an unrelated
+    stream nor is recorded in it."""
+    report("tiled_capture")
+    g, one = (_solver(hip, (57, 9), "fp32", "cavity") for _ in range(2))
+    rt = C.CDLL("libamdhip64.so.7")
+    stream, graph, nodes = C.c_void_p(), C.c_void_p(), C.c_size_t(99)
+    rt.hipStreamDestroy.argtypes = rt.hipGraphDestroy.argtypes = [C.c_void_p]
+    assert rt.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+    g.wait()
+    one.wait()
+    assert rt.hipStreamBeginCapture(stream, 0) == 0  # hipStreamCaptureModeGlobal
+    before = g.resident_bytes()
+    g.step(8)
+    assert rt.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert rt.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and nodes.value == 0
+    assert rt.hipGraphDestroy(graph) == 0 and rt.hipStreamDestroy(stream) == 0
+    assert g.resident_bytes() >= before + g.population_bytes()
+    for _ in range(8):
+        one.step(1)
+    for got, want in zip(_state(g), _state(one)):
+        assert np.array_equal(got, want)
