@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <mutex>
 #include <stdexcept>
@@ -34,8 +35,6 @@ class WorkspacePool {
 
     // A block of at least `bytes` on the current device, for the caller alone until put().
     unsigned char* take(size_t bytes, size_t* got);
-    // The same from the idle blocks only; null if none fits.
-    unsigned char* take_idle(size_t bytes, size_t* got);
     // Ends the use of a block of the current device; no work that uses it is pending.
     void put(unsigned char* ptr, size_t bytes, bool keep);
     // Bytes of the idle blocks on the current device.
@@ -77,6 +76,9 @@ class WorkspacePool {
             if (b.device == device) sum += b.bytes;
         return sum;
     }
+    size_t held_bytes_locked(int device) const;
+    // The smallest idle block of the device with `bytes` to `most` bytes, no longer idle; null if none.
+    unsigned char* take_idle_locked(int device, size_t bytes, size_t most, size_t* got);
     // Frees the oldest idle blocks of the device until at most `limit` bytes are idle.
     bool trim_locked(int device, size_t limit) {
         bool any = false;
@@ -142,7 +144,10 @@ class HeldBlock {
         const std::lock_guard<std::mutex> lock(WorkspacePool::instance().mutex_);
         busy_ = false;
     }
-    size_t bytes() const { return bytes_; }
+    size_t bytes() const {
+        const std::lock_guard<std::mutex> lock(WorkspacePool::instance().mutex_);
+        return bytes_;
+    }
 
   private:
     friend class WorkspacePool;
@@ -185,13 +190,17 @@ inline hipError_t device_malloc(void** p, size_t bytes) {
     return hipMalloc(p, bytes);
 }
 
-inline unsigned char* WorkspacePool::take_idle(size_t bytes, size_t* got) {
-    // The smallest idle block that holds the request, unless it would waste more than half of it.
-    const std::lock_guard<std::mutex> lock(mutex_);
-    const int device = current_device();
+inline size_t WorkspacePool::held_bytes_locked(int device) const {
+    size_t sum = 0;
+    for (const HeldBlock* h : held_)
+        if (h->device_ == device) sum += h->bytes_;
+    return sum;
+}
+
+inline unsigned char* WorkspacePool::take_idle_locked(int device, size_t bytes, size_t most, size_t* got) {
     size_t best = idle_.size();
     for (size_t k = 0; k < idle_.size(); ++k)
-        if (idle_[k].device == device && idle_[k].bytes >= bytes && idle_[k].bytes / 2 <= bytes &&
+        if (idle_[k].device == device && idle_[k].bytes >= bytes && idle_[k].bytes <= most &&
             (best == idle_.size() || idle_[k].bytes < idle_[best].bytes))
             best = k;
     if (best == idle_.size()) return nullptr;
@@ -202,7 +211,10 @@ inline unsigned char* WorkspacePool::take_idle(size_t bytes, size_t* got) {
 }
 
 inline unsigned char* WorkspacePool::take(size_t bytes, size_t* got) {
-    if (unsigned char* const p = take_idle(bytes, got)) return p;
+    {  // an idle block, unless it would waste more than half of it
+        const std::lock_guard<std::mutex> lock(mutex_);
+        if (unsigned char* const p = take_idle_locked(current_device(), bytes, 2 * bytes + 1, got)) return p;
+    }
     void* p = nullptr;
     if (const hipError_t e = device_malloc(&p, bytes); e != hipSuccess)
         throw std::runtime_error(std::string("hipMalloc: ") + hipGetErrorString(e));
@@ -233,36 +245,44 @@ inline unsigned char* HeldBlock::take(size_t bytes) {
             return ptr_;
         }
         if (refused_) return nullptr;
-        size_t sum = bytes;
         const int device = WorkspacePool::current_device();
-        for (const HeldBlock* h : pool.held_)
-            if (h->device_ == device) sum += h->bytes_;
-        if (sum > WorkspacePool::bound()) return nullptr;
-    }
-    size_t got = 0;
-    unsigned char* p = pool.take_idle(bytes, &got);
-    if (!p) {  // a plain hipMalloc: what the caller can do without takes no block from another owner
-        const AllocationDuringCapture permit;  // a caller that steps expects no allocation
-        void* fresh = nullptr;
-        if (hipMalloc(&fresh, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            refused_ = true;
+        const size_t held = pool.held_bytes_locked(device), bound = WorkspacePool::bound();
+        if (held > bound || bytes > bound - held) return nullptr;
+        try {
+            pool.held_.push_back(this);
+        } catch (...) {  // no host memory for the list
             return nullptr;
         }
-        p = static_cast<unsigned char*>(fresh);
-        got = bytes;
+        // Entered before the allocation, so that the next one to ask counts it.  An idle block is held
+        // whole: only one of nearly the size that fits the bound too.
+        device_ = device;
+        bytes_ = bytes;
+        busy_ = true;
+        size_t got = 0;
+        if (unsigned char* const p =
+                pool.take_idle_locked(device, bytes, std::min(bytes + bytes / 8, bound - held), &got)) {
+            ptr_ = p;
+            bytes_ = got;
+            return ptr_;
+        }
+    }
+    // A plain hipMalloc: what the caller can do without takes no block from another owner.
+    void* fresh = nullptr;
+    hipError_t e;
+    {
+        const AllocationDuringCapture permit;  // a caller that steps expects no allocation
+        e = hipMalloc(&fresh, bytes);
     }
     const std::lock_guard<std::mutex> lock(pool.mutex_);
-    try {
-        pool.held_.push_back(this);
-    } catch (...) {  // no host memory for the list
-        (void)hipFree(p);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        refused_ = true;
+        forget(pool);
+        bytes_ = 0;
+        busy_ = false;
         return nullptr;
     }
-    ptr_ = p;
-    bytes_ = got;
-    device_ = WorkspacePool::current_device();
-    busy_ = true;
+    ptr_ = static_cast<unsigned char*>(fresh);
     return ptr_;
 }
 

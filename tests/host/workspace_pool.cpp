@@ -72,13 +72,58 @@ void foreign_capture() {
     pool.leave();
 }
 
+void held_bound() {
+    pool.enter();
+    leave_idle(90);
+    HeldBlock small;
+    EXPECT(small.take(60));  // not the idle block: half as much again would be held
+    EXPECT(small.bytes() == 60 && pool.idle_bytes() == 90);
+    HeldBlock near, over;
+    EXPECT(near.take(38));  // 98 of 100 held
+    EXPECT(!over.take(3));
+    near.done();
+    pool.leave();
+}
+
+void held_close_fit() {
+    pool.enter();
+    unsigned char* const idle = leave_idle(88);
+    HeldBlock h;
+    EXPECT(h.take(80) == idle && h.bytes() == 88 && pool.idle_bytes() == 0);
+    pool.leave();
+}
+
+void held_close_fit_over_the_bound() {
+    pool.enter();
+    leave_idle(54);
+    HeldBlock first, second;
+    EXPECT(first.take(48) && first.bytes() == 54);
+    leave_idle(54);
+    EXPECT(second.take(46) && second.bytes() == 46);  // 54 + 54 is more than 100
+    EXPECT(pool.idle_bytes() == 54);
+    pool.leave();
+}
+
+void held_bound_two_threads() {
+    pool.enter();
+    HeldBlock a, b;
+    unsigned char* other = nullptr;
+    stub::during_malloc = [&] { other = b.take(60); };  // what a second thread does meanwhile
+    EXPECT(a.take(60));
+    EXPECT(!other && stub::used == 60);
+    pool.leave();
+}
+
 }  // namespace
 
 int main(int, char** argv) {
     const struct {
         const char* name;
         void (*run)();
-    } all[] = {{"reuse", reuse}, {"full_device", full_device}, {"foreign_capture", foreign_capture}};
+    } all[] = {{"reuse", reuse}, {"full_device", full_device}, {"foreign_capture", foreign_capture},
+                 {"held_bound", held_bound}, {"held_close_fit", held_close_fit},
+                 {"held_close_fit_over_the_bound", held_close_fit_over_the_bound},
+                 {"held_bound_two_threads", held_bound_two_threads}};
     for (const auto& s : all)
         if (std::strcmp(argv[1], s.name) == 0) return s.run(), 0;
     return 2;
