@@ -162,7 +162,10 @@ class HeldBlock {
     size_t bytes_ = 0;
     int device_ = 0;
     bool busy_ = false;
-    bool refused_ = false;  // the device was full once: not tried again
+    // Takes still to pass before a device that was full is asked again: another owner may have freed
+    // memory by then, and a failing hipMalloc at every call is not worth its time.
+    static constexpr unsigned kPause = 255;
+    unsigned pause_ = 0;
 };
 
 inline bool WorkspacePool::trim() {
@@ -244,7 +247,10 @@ inline unsigned char* HeldBlock::take(size_t bytes) {
             busy_ = true;
             return ptr_;
         }
-        if (refused_) return nullptr;
+        if (pause_ > 0) {
+            --pause_;
+            return nullptr;
+        }
         const int device = WorkspacePool::current_device();
         const size_t held = pool.held_bytes_locked(device), bound = WorkspacePool::bound();
         if (held > bound || bytes > bound - held) return nullptr;
@@ -276,7 +282,7 @@ inline unsigned char* HeldBlock::take(size_t bytes) {
     const std::lock_guard<std::mutex> lock(pool.mutex_);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        refused_ = true;
+        if (e == hipErrorOutOfMemory) pause_ = kPause;
         forget(pool);
         bytes_ = 0;
         busy_ = false;

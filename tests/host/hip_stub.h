@@ -7,14 +7,14 @@
 #include <functional>
 #include <map>
 
-enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorStreamCaptureUnsupported = 900 };
+enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorUnknown = 999, hipErrorStreamCaptureUnsupported = 900 };
 enum hipStreamCaptureMode { hipStreamCaptureModeGlobal, hipStreamCaptureModeThreadLocal, hipStreamCaptureModeRelaxed };
 
 namespace stub {
 inline size_t capacity = 1600, used = 0, frees = 0, mallocs = 0;
 inline uintptr_t next = 0x1000;
 inline std::map<void*, size_t> live;
-inline bool capturing = false, broken = false;
+inline bool capturing = false, broken = false, fail_next = false;
 inline hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
 inline std::function<void()> during_malloc;  // run once, inside the next hipMalloc
 }  // namespace stub
@@ -29,6 +29,10 @@ inline hipError_t hipMalloc(void** p, size_t bytes) {
     if (stub::capturing && stub::mode != hipStreamCaptureModeRelaxed) {
         stub::broken = true;
         return hipErrorStreamCaptureUnsupported;
+    }
+    if (stub::fail_next) {
+        stub::fail_next = false;
+        return hipErrorUnknown;
     }
     if (bytes > stub::capacity - stub::used) return hipErrorOutOfMemory;
     stub::used += bytes;

@@ -114,6 +114,30 @@ void held_bound_two_threads() {
     pool.leave();
 }
 
+void held_again_after_a_full_device() {
+    pool.enter();
+    void* all = nullptr;
+    EXPECT(hipMalloc(&all, stub::capacity) == hipSuccess);
+    HeldBlock h;
+    const size_t before = stub::mallocs;
+    for (int k = 0; k < 10; ++k) EXPECT(!h.take(60));
+    EXPECT(stub::mallocs == before + 1);  // a full device is not asked at every call
+    (void)hipFree(all);
+    int calls = 0;
+    while (!h.take(60) && calls < 1000) ++calls;
+    EXPECT(calls < 300 && h.bytes() == 60);
+    pool.leave();
+}
+
+void held_again_after_a_failed_call() {
+    pool.enter();
+    HeldBlock h;
+    stub::fail_next = true;
+    EXPECT(!h.take(60));
+    EXPECT(h.take(60));  // not a full device: asked again at the next call
+    pool.leave();
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -123,7 +147,9 @@ int main(int, char** argv) {
     } all[] = {{"reuse", reuse}, {"full_device", full_device}, {"foreign_capture", foreign_capture},
                  {"held_bound", held_bound}, {"held_close_fit", held_close_fit},
                  {"held_close_fit_over_the_bound", held_close_fit_over_the_bound},
-                 {"held_bound_two_threads", held_bound_two_threads}};
+                 {"held_bound_two_threads", held_bound_two_threads},
+                 {"held_again_after_a_full_device", held_again_after_a_full_device},
+                 {"held_again_after_a_failed_call", held_again_after_a_failed_call}};
     for (const auto& s : all)
         if (std::strcmp(argv[1], s.name) == 0) return s.run(), 0;
     return 2;
