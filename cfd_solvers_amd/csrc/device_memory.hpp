@@ -42,6 +42,13 @@ class WorkspacePool {
         const std::lock_guard<std::mutex> lock(mutex_);
         return idle_bytes_locked(current_device());
     }
+    // What trim() would give back: the current device's idle blocks and the held ones that no call is
+    // using.  A budget of the device's memory counts them as free.
+    size_t reclaimable_bytes() {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        const int device = current_device();
+        return idle_bytes_locked(device) + held_bytes_locked(device, false);
+    }
     // Gives back the current device's idle blocks and the held ones that no call is using; false if
     // there were none.
     bool trim();
@@ -76,7 +83,7 @@ class WorkspacePool {
             if (b.device == device) sum += b.bytes;
         return sum;
     }
-    size_t held_bytes_locked(int device) const;
+    size_t held_bytes_locked(int device, bool busy_too) const;
     // The smallest idle block of the device with `bytes` to `most` bytes, no longer idle; null if none.
     unsigned char* take_idle_locked(int device, size_t bytes, size_t most, size_t* got);
     // Frees the oldest idle blocks of the device until at most `limit` bytes are idle.
@@ -193,10 +200,10 @@ inline hipError_t device_malloc(void** p, size_t bytes) {
     return hipMalloc(p, bytes);
 }
 
-inline size_t WorkspacePool::held_bytes_locked(int device) const {
+inline size_t WorkspacePool::held_bytes_locked(int device, bool busy_too) const {
     size_t sum = 0;
     for (const HeldBlock* h : held_)
-        if (h->device_ == device) sum += h->bytes_;
+        if (h->device_ == device && (busy_too || !h->busy_)) sum += h->bytes_;
     return sum;
 }
 
@@ -252,7 +259,7 @@ inline unsigned char* HeldBlock::take(size_t bytes) {
             return nullptr;
         }
         const int device = WorkspacePool::current_device();
-        const size_t held = pool.held_bytes_locked(device), bound = WorkspacePool::bound();
+        const size_t held = pool.held_bytes_locked(device, true), bound = WorkspacePool::bound();
         if (held > bound || bytes > bound - held) return nullptr;
         try {
             pool.held_.push_back(this);

@@ -980,7 +980,7 @@ struct cfd_lbm_solver {
         const size_t fixed = pop_elems * real + 2 * cells * 8 + 8 * 4096;  // with the padding and sums below
         size_t free_b = 0, total_b = 0;
         hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-        free_b += cfd_hip::WorkspacePool::instance().idle_bytes();  // given back on demand
+        free_b += cfd_hip::WorkspacePool::instance().reclaimable_bytes();  // given back on demand
         size_t buffers = 0;  // state buffers besides f
         if (every > 0) {
             buffers = static_cast<size_t>((steps + every - 1) / every + std::min<uint64_t>(every, steps) - 1);

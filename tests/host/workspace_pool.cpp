@@ -138,6 +138,20 @@ void held_again_after_a_failed_call() {
     pool.leave();
 }
 
+void reclaimable() {
+    pool.enter();
+    HeldBlock busy, rests;
+    EXPECT(busy.take(30) && rests.take(50));
+    rests.done();
+    leave_idle(90);
+    EXPECT(pool.reclaimable_bytes() == 140);
+    // What a caller counts on is there: free memory and the reclaimable bytes in one block.
+    void* p = nullptr;
+    EXPECT(cfd_hip::device_malloc(&p, stub::capacity - stub::used + 140) == hipSuccess);
+    EXPECT(pool.reclaimable_bytes() == 0);
+    pool.leave();
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -149,7 +163,8 @@ int main(int, char** argv) {
                  {"held_close_fit_over_the_bound", held_close_fit_over_the_bound},
                  {"held_bound_two_threads", held_bound_two_threads},
                  {"held_again_after_a_full_device", held_again_after_a_full_device},
-                 {"held_again_after_a_failed_call", held_again_after_a_failed_call}};
+                 {"held_again_after_a_failed_call", held_again_after_a_failed_call},
+                 {"reclaimable", reclaimable}};
     for (const auto& s : all)
         if (std::strcmp(argv[1], s.name) == 0) return s.run(), 0;
     return 2;
