@@ -5,13 +5,13 @@ in ``include/cfd_lbm/c_api.h``); this package is the ctypes host layer over it, 
 reference's ``python/cfd_solvers`` bindings.  Build the library with
 ``python -m cfd_solvers_amd.build``.
 """
-from .bindings import (EsotericPullHipSolver, MacroscopicFields, SolverLibrary, load, checkpoint_plan, FLUID,
-                       VELOCITY_INLET, PRESSURE_OUTLET, WALL, LATTICES, STORAGE, OBJECTIVES, voxelize_surface,
+from .bindings import (EsotericPullHipSolver, MacroscopicFields, SolverLibrary, load, checkpoint_plan,
+                       release_workspaces, FLUID, VELOCITY_INLET, PRESSURE_OUTLET, WALL, LATTICES, STORAGE, OBJECTIVES, voxelize_surface,
                        voxelize_timing, transform_surface, ResidentThermalD3Q7, ResidentFreeSurface,
                        ResidentParticles, ResidentFlowDiagnostics)
 
-__all__ = ["EsotericPullHipSolver", "MacroscopicFields", "SolverLibrary", "load", "checkpoint_plan", "FLUID",
-           "VELOCITY_INLET", "PRESSURE_OUTLET", "WALL", "LATTICES", "STORAGE", "OBJECTIVES", "voxelize_surface",
+__all__ = ["EsotericPullHipSolver", "MacroscopicFields", "SolverLibrary", "load", "checkpoint_plan",
+           "release_workspaces", "FLUID", "VELOCITY_INLET", "PRESSURE_OUTLET", "WALL", "LATTICES", "STORAGE", "OBJECTIVES", "voxelize_surface",
            "voxelize_timing", "transform_surface", "ResidentThermalD3Q7", "ResidentFreeSurface",
            "ResidentParticles", "ResidentFlowDiagnostics"]
 

@@ -38,6 +38,9 @@ class LbmAdjointProblem:
     ``checkpoint_every == 0`` selects binomial checkpointing with ``snapshots`` state buffers
     (0: as many as fit in device memory).  ``objective`` is ``"pressure_drop"`` (planes ``x_in``,
     ``x_out``) or ``"drag"`` (``body``: nonzero on the wall cells of the body, along ``drag_axis``).
+
+    A run's working memory of up to 1/16 of the device's is kept for the next run;
+    ``cfd_solvers_amd.release_workspaces()`` gives it back to PyTorch's allocator.
     """
 
     flags: np.ndarray

@@ -48,6 +48,7 @@ _SIGNATURES = {
     "cfd_lbm_set_porosity": [C.c_void_p, C.c_void_p],
     "cfd_lbm_set_inlet_outlet": [C.c_void_p, C.c_float, C.c_float],
     "cfd_lbm_set_local_acceleration": [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p],
+    "cfd_lbm_release_workspaces": [],
     "cfd_lbm_step": [C.c_void_p, C.c_uint64],
     "cfd_lbm_step_timed": [C.c_void_p, C.c_uint64, C.POINTER(C.c_float)],
     "cfd_lbm_synchronize": [C.c_void_p],
@@ -506,6 +507,13 @@ class EsotericPullHipSolver:
         store = np.empty(self.q * self.cells, dtype=np.int64)
         self.lib.call("cfd_lbm_index_map", self._h, parity, load, store)
         return load.reshape(self.q, self.cells), store.reshape(self.q, self.cells)
+
+
+def release_workspaces(library=None):
+    """Gives back the device memory that the library keeps for later calls (the working memory of
+    finished adjoint runs, the second lattices of D2Q9 solvers), for the sake of other allocators in the
+    process: PyTorch's cannot reclaim it.  The next call that wants it allocates again."""
+    load(library).call("cfd_lbm_release_workspaces")
 
 
 def checkpoint_plan(steps, snapshots, library=None):

@@ -6,7 +6,8 @@
 // from WorkspacePool (Workspace), which keeps the blocks of finished calls for the next one, of
 // whichever solver; a block that one object wants at every call it holds itself (HeldBlock).  Neither
 // holds a state between calls.  Idle and held blocks are each bounded to 1 / kKeptFraction of the
-// device's memory, and both are given back before any allocation of this library fails.
+// device's memory, and both are given back before any allocation of this library fails, with the last
+// solver, or at cfd_lbm_release_workspaces: other allocators cannot reclaim them.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -52,6 +53,8 @@ class WorkspacePool {
     // Gives back the current device's idle blocks and the held ones that no call is using; false if
     // there were none.
     bool trim();
+    // trim() on every device that has blocks.
+    void release();
     // Users (solvers) alive; the last one to leave gives back every idle block.
     void enter() {
         const std::lock_guard<std::mutex> lock(mutex_);
@@ -189,6 +192,21 @@ inline bool WorkspacePool::trim() {
         any = true;
     }
     return any;
+}
+
+inline void WorkspacePool::release() {
+    std::vector<int> devices;
+    {
+        const std::lock_guard<std::mutex> lock(mutex_);
+        for (const Block& b : idle_) devices.push_back(b.device);
+        for (const HeldBlock* h : held_) devices.push_back(h->device_);
+    }
+    std::sort(devices.begin(), devices.end());
+    devices.erase(std::unique(devices.begin(), devices.end()), devices.end());
+    const int before = current_device();
+    for (const int d : devices)
+        if (hipSetDevice(d) == hipSuccess) (void)trim();
+    if (!devices.empty()) (void)hipSetDevice(before);
 }
 
 // hipMalloc on the current device; when that finds the device full, once more after the idle

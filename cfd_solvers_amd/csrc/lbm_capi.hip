@@ -1444,6 +1444,10 @@ extern "C" {
 
 const char* cfd_lbm_version(void) { return "cfd_lbm_hip 0.1.0 (gfx950)"; }
 
+int cfd_lbm_release_workspaces(char* error, size_t cap) {
+    return guarded(error, cap, [] { cfd_hip::WorkspacePool::instance().release(); });
+}
+
 int cfd_lbm_create(int lattice, size_t nx, size_t ny, size_t nz, float tau, float ax, float ay, float az, int storage,
                    cfd_lbm_solver** out, char* error, size_t cap) {
     return guarded(error, cap, [&] {

@@ -59,6 +59,12 @@ enum {
 };
 
 CFD_LBM_API const char* cfd_lbm_version(void);
+/* Gives back the device memory that the library keeps for later calls: the working memory of
+ * finished adjoint runs and the second lattices of D2Q9 solvers (each up to 1/16 of a device's
+ * memory while solvers are alive).  Allocations of this library reclaim it by themselves; other
+ * allocators in the process cannot.  Nothing is lost: the next call that wants it allocates again.
+ * May be called from any thread; waits for the devices' pending work. */
+CFD_LBM_API int cfd_lbm_release_workspaces(char* error, size_t error_capacity);
 
 /* EsotericPullSolver(InPlaceLbmConfig) -- esoteric_pull.hpp:109-115,292-302.  Throws (returns 1)
  * if tau <= 0.5, nx or ny < 2, nz < 2 for 3-D lattices.  nz is forced to 1 for D2Q9.  The

@@ -1,4 +1,4 @@
-// A host-only stand-in for the few HIP calls of device_memory.hpp: one device of `capacity` bytes whose
+// A host-only stand-in for the few HIP calls of device_memory.hpp: devices of `capacity` bytes together, whose
 // blocks are host addresses, and a capture on some other stream that an unguarded allocation breaks.
 #pragma once
 
@@ -13,6 +13,7 @@ enum hipStreamCaptureMode { hipStreamCaptureModeGlobal, hipStreamCaptureModeThre
 namespace stub {
 inline size_t capacity = 1600, used = 0, frees = 0, mallocs = 0;
 inline uintptr_t next = 0x1000;
+inline int device = 0;
 inline std::map<void*, size_t> live;
 inline bool capturing = false, broken = false, fail_next = false;
 inline hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
@@ -46,7 +47,8 @@ inline hipError_t hipFree(void* p) {
     stub::live.erase(p);
     return hipSuccess;
 }
-inline hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+inline hipError_t hipGetDevice(int* d) { return *d = stub::device, hipSuccess; }
+inline hipError_t hipSetDevice(int d) { return stub::device = d, hipSuccess; }
 inline hipError_t hipDeviceTotalMem(size_t* total, int) { return *total = stub::capacity, hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline const char* hipGetErrorString(hipError_t) { return "stub"; }

@@ -152,6 +152,23 @@ void reclaimable() {
     pool.leave();
 }
 
+void release() {
+    pool.enter();
+    HeldBlock busy, rests;
+    EXPECT(busy.take(30) && rests.take(40));
+    rests.done();
+    leave_idle(50);
+    stub::device = 1;
+    leave_idle(60);
+    stub::device = 2;
+    EXPECT(stub::used == 180);
+    pool.release();
+    EXPECT(stub::used == 30 && stub::device == 2);  // the block in use stays
+    stub::device = 0;
+    EXPECT(rests.take(40) && leave_idle(50));
+    pool.leave();
+}
+
 }  // namespace
 
 int main(int, char** argv) {
@@ -164,7 +181,8 @@ int main(int, char** argv) {
                  {"held_bound_two_threads", held_bound_two_threads},
                  {"held_again_after_a_full_device", held_again_after_a_full_device},
                  {"held_again_after_a_failed_call", held_again_after_a_failed_call},
-                 {"reclaimable", reclaimable}};
+                 {"reclaimable", reclaimable},
+                 {"release", release}};
     for (const auto& s : all)
         if (std::strcmp(argv[1], s.name) == 0) return s.run(), 0;
     return 2;

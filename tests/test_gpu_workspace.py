@@ -74,3 +74,35 @@ def test_two_level_plans_agree(hip, every):
     report("two_level_plan", every=every)
     s = _solver(hip, (19, 14, 12), "fp32")
     assert _same(_run(s, every, 0), _run(s, 0, 3))
+
+
+def test_release(hip):
+    """Kept memory goes back to the device on request, and the next calls return what they returned."""
+    import ctypes as C
+
+    report("workspace_release")
+    rt = C.CDLL("libamdhip64.so.7")
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    s = _solver(hip, (33, 40, 41), "fp32")
+    flow = hip.EsotericPullHipSolver("d2q9", 2048, 1024, 1, 0.6)
+    flow.initialize_taylor_green(0.02, 1e-4, 3)
+    want = _run(s, 4, 0)
+    flow.step(16)
+    fields = flow.download_macroscopic()
+    before, held = free_bytes(), flow.resident_bytes()
+    hip.release_workspaces()
+    assert flow.resident_bytes() <= held - flow.population_bytes()
+    assert free_bytes() >= before + flow.population_bytes()
+    assert _same(_run(s, 4, 0), want)
+    flow.initialize_taylor_green(0.02, 1e-4, 3)
+    flow.step(16)
+    again = flow.download_macroscopic()
+    assert flow.resident_bytes() == held
+    assert np.array_equal(again.rho, fields.rho) and np.array_equal(again.ux, fields.ux)
+    flow.close()
+    s.close()

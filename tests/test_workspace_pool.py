@@ -23,7 +23,7 @@ def program(tmp_path_factory):
 @pytest.mark.parametrize("scenario", ["reuse", "full_device", "foreign_capture", "held_bound", "held_close_fit",
                                       "held_close_fit_over_the_bound", "held_bound_two_threads",
                                       "held_again_after_a_full_device", "held_again_after_a_failed_call",
-                                      "reclaimable"])
+                                      "reclaimable", "release"])
 def test_pool(program, scenario):
     r = subprocess.run([str(program), scenario], capture_output=True, text=True, timeout=30)
     assert r.returncode == 0, r.stderr
