@@ -530,9 +530,13 @@ __global__ void __launch_bounds__(kBlock) vof_curvature_tension(const float* __r
         const float ox = ld(ax, n), oy = ld(ay, n), oz = ld(az, n);
         el(geo + 3 * static_cast<size_t>(d.cells), n) = kappa;
         const float c = sigma * kappa / density;
-        el(ax, n) = ox + c * gx;
-        el(ay, n) = oy + c * gy;
-        el(az, n) = oz + c * gz;
+        // One plane may serve several axes: it then takes their terms one after another.
+        const float vx = ox + c * gx;
+        const float vy = (ay == ax ? vx : oy) + c * gy;
+        const float vz = (az == ay ? vy : az == ax ? vx : oz) + c * gz;
+        el(ax, n) = vx;
+        el(ay, n) = vy;
+        el(az, n) = vz;
     });
 }
 
@@ -1087,7 +1091,7 @@ int cfd_lbm_surface_add_surface_tension(cfd_lbm_surface* s, float* ax, float* ay
         vof_normals<<<normals.grid, normals.block, 0, s->flow.stream>>>(s->fill, s->geometry, s->dims);
         vof_curvature_tension<<<sh.grid, sh.block, 0, s->flow.stream>>>(s->fill, s->geometry, ax, ay, az, s->dims,
                                                                         surface_tension, density);
-        check(hipGetLastError(), "vof_tension");
+        check(hipGetLastError(), "vof_curvature_tension");
     });
 }
 int cfd_lbm_surface_volume(cfd_lbm_surface* s, double* volume, char* error, size_t cap) {

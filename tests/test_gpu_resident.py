@@ -267,3 +267,27 @@ def test_module_errors(hip):
     s.close()
     p.close()
     flow.close()
+
+
+@pytest.mark.parametrize("planes", [(0, 0, 1), (0, 1, 0), (0, 1, 1), (0, 0, 0)])
+def test_surface_tension_into_shared_planes(hip, planes):
+    """A plane passed for several axes takes the axes' terms in turn, x first."""
+    report("tension_shared", planes=planes)
+    flow = flow_with_motion(hip, 24, 20, 18)
+    z, y, x = np.meshgrid(*(np.arange(n) for n in flow.shape), indexing="ij")
+    d = np.sqrt((x - 11.3) ** 2 + (y - 9.6) ** 2 + (z - 8.2) ** 2)
+    s = hip.ResidentFreeSurface(flow)
+    s.upload_fill((0.5 * (1 - np.tanh((d - 6.0) / 1.5))).astype(np.float32))
+    force = flow.device_local_acceleration(True)
+    s.add_surface_tension_acceleration(force, 0.072, 1.3)
+    terms = [flow.device_download(p) for p in force]  # onto zeros: the terms themselves
+    assert all(t.any() for t in terms)
+    force = flow.device_local_acceleration(True)
+    s.add_surface_tension_acceleration(tuple(force[k] for k in planes), 0.072, 1.3)
+    want = [np.zeros(flow.cells, np.float32) for _ in range(3)]
+    for term, k in zip(terms, planes):
+        want[k] = want[k] + term
+    for p, w in zip(force, want):
+        assert np.array_equal(flow.device_download(p), w)
+    s.close()
+    flow.close()
