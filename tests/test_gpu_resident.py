@@ -291,3 +291,43 @@ def test_surface_tension_into_shared_planes(hip, planes):
         assert np.array_equal(flow.device_download(p), w)
     s.close()
     flow.close()
+
+
+def test_many_particles_match_oracle(hip, oracle_mod):
+    """5000 particles: 20 blocks, so each XCD takes a run of two, four blocks are left over and the last
+    wavefront is partial; one-way bit for bit, the reactions to the order of the atomic sums."""
+    report("many_particles")
+    flow = flow_with_motion(hip)
+    macro = flow.refresh_device_macroscopic()
+    u = velocity(flow, macro)
+    r = oracle_mod.Resident(flow.nx, flow.ny, flow.nz)
+    rng = np.random.default_rng(11)
+    n = 5000
+    p = np.column_stack([rng.uniform(-3, flow.nx + 3, n), rng.uniform(0, flow.ny, n), rng.uniform(0, flow.nz, n),
+                         rng.normal(scale=0.01, size=(n, 3)), rng.uniform(0.5, 2, n), rng.uniform(0.2, 1, n)])
+    parts = hip.ResidentParticles(flow, n)
+    parts.upload(p)
+    force = flow.device_local_acceleration(True)
+    want = p.astype(np.float32).astype(np.float64)
+    zero = np.zeros((3,) + flow.shape)
+    for _ in range(3):
+        parts.advance(macro, force, 0.05, False, (0.0, -0.01, 0.0))
+        want, _ = r.particles_advance(want, u, zero, 0.05, False, (0.0, -0.01, 0.0))
+    assert np.array_equal(parts.download(), want)
+    parts.advance(macro, force, 0.05, True)
+    got_a = np.stack([flow.device_download(q).reshape(flow.shape) for q in force])
+    want_p, want_a = r.particles_advance(want, u, zero, 0.05, True)
+    assert np.array_equal(parts.download(), want_p)
+    # A cell sums the terms of the particles in the 8 cells around it, m at most, of magnitude D at most
+    # (mass <= 2 and response >= 0.2); in any order a float sum is off by less than m units of 2^-24 of
+    # the sum of the magnitudes, and two orders differ by twice that.
+    cell = np.floor(want[:, :3]).astype(int) % (flow.nx, flow.ny, flow.nz)
+    m = np.zeros((flow.nx, flow.ny, flow.nz), int)
+    np.add.at(m, tuple(cell.T), 1)
+    for axis in range(3):
+        m = m + np.roll(m, 1, axis)
+    D = 2.0 / 0.2 * (np.abs(u).max() + np.abs(want[:, 3:6]).max())
+    assert np.abs(want_a).max() > 0
+    assert np.abs(got_a - want_a).max() <= 2 * m.max() * 2.0 ** -24 * m.max() * D
+    parts.close()
+    flow.close()
