@@ -1258,11 +1258,15 @@ struct cfd_lbm_solver {
         hip_check(hipGetLastError(), "zero_words");
     }
 
-    // The second lattice if `count` steps may run several to a launch (lbm_tiled.hip): an unporous D2Q9
-    // lattice whose second copy is within the workspace bound, outside of stream capture (a graph is
-    // replayed on `f` alone, and it must not hold an allocation).  Null: single steps.
+    bool forced() const { return ax != 0.0F || ay != 0.0F || az != 0.0F || static_cast<bool>(lacc) || les; }
+    // Whether pairs of launches of `k` steps each are the faster way for this lattice (lbm_tiled.hip).
+    bool tiled(int k) const { return !gamma && cfd_hip::tiled_pays(q, storage, nx, ny, f.bytes, k, bounded(), forced()); }
+
+    // The second lattice if `count` steps run several to a launch: its copy is within the workspace bound,
+    // and not during stream capture (a graph is replayed on `f` alone, and it must not hold an
+    // allocation).  Null: single steps.
     unsigned char* second_lattice(uint64_t count) {
-        if (count < 4U || gamma || !cfd_hip::tiled_supported(q, storage, nx, ny)) return nullptr;
+        if (!(count >= 8U && tiled(4)) && !(count >= 4U && tiled(2))) return nullptr;
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
         return second.take(f.bytes);
@@ -1271,10 +1275,10 @@ struct cfd_lbm_solver {
     void step(uint64_t count) {
         use_device();
         const bool b = bounded();
-        const bool forced = ax != 0.0F || ay != 0.0F || az != 0.0F || static_cast<bool>(lacc) || les;
+        const bool with_force = forced();
         LaunchState st = state();
         const auto single = [&] {
-            ops->step(st, odd(), b, forced, f.ptr, f.ptr);
+            ops->step(st, odd(), b, with_force, f.ptr, f.ptr);
             ++t;
             --count;
         };
@@ -1286,9 +1290,9 @@ struct cfd_lbm_solver {
             if (odd()) single();  // the tiled kernels start at even parity
             // Pairs of launches, f to the second lattice and back.
             for (int k = 4; k >= 2; k -= 2)
-                for (; count >= 2U * static_cast<uint64_t>(k); count -= 2U * static_cast<uint64_t>(k)) {
-                    cfd_hip::tiled_steps(storage, st, k, b, forced, f.ptr, other);
-                    cfd_hip::tiled_steps(storage, st, k, b, forced, other, f.ptr);
+                for (; tiled(k) && count >= 2U * static_cast<uint64_t>(k); count -= 2U * static_cast<uint64_t>(k)) {
+                    cfd_hip::tiled_steps(storage, st, k, b, with_force, f.ptr, other);
+                    cfd_hip::tiled_steps(storage, st, k, b, with_force, other, f.ptr);
                     t += 2U * static_cast<uint64_t>(k);
                 }
         }

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(W* Rows) void tiled_step(const void* __restrict__ s
 constexpr uint32_t kHalo = 4;  // the largest K
 
 // Two tiles, both 64 slots (one wavefront) wide.  34 rows (FP32: 77 KiB of LDS, two blocks a CU)
-// recompute 17 % of the cells at K = 4 and are bound by the vector units: 4096^2 cavity FP32 134 us a
+// recompute 18 % of the cells at K = 4 and are bound by the vector units: 4096^2 cavity FP32 134 us a
 // step against 201 single (periodic 127 against 201, FP16S 91 against 115), 1400^2 15.1 against 26.2.
 // 26 rows measure 137-142, 42 rows 152, 8 rows of threads instead of 16 139.
 //
@@ -169,6 +169,7 @@ constexpr uint32_t kHalo = 4;  // the largest K
 // the large tile; 330^2: 2.2; 400^2: 2.6 against 5.5 and 3.0; 100 x 500: 1.9.  Tiles of 32 x 16 slots
 // measure 2.1, 2.4, 2.9 and 2.1; the large tile is ahead at 600^2 (3.6 against 4.6).
 constexpr uint32_t kLargeTileCells = 200000U;
+constexpr uint32_t kLargeRows = 34U - 2U * kHalo;  // interior rows of the large tile
 
 // Interior rows (2 to `most`) of tiles with `strips` columns: blocks are dealt to 256 CUs, and a block
 // issues K rows + K (K - 1) wavefronts over its levels (rows + 2 (K - s) at level s).
@@ -194,8 +195,10 @@ template <class T, bool Bounded, bool Forced, int K> void launch(const LaunchSta
         hipLaunchKernelGGL(kernel, dim3(tx * ((st.geo.ny + rows - 1U) / rows)), dim3(threads), 0, st.stream, src, dst,
                            st.geo, *static_cast<const Physics<Real>*>(st.physics), tx, rows);
     };
-    if (st.cells >= kLargeTileCells) go(tiled_step<T, Bounded, Forced, K, 34, 16>, 34U - 2U * K, 1024U);
-    else go(tiled_step<T, Bounded, Forced, K, 16, 12>, tile_rows(tx, st.geo.ny, K, 16U - 2U * K), 768U);
+    if (st.cells < kLargeTileCells)
+        go(tiled_step<T, Bounded, Forced, K, 16, 12>, tile_rows(tx, st.geo.ny, K, 16U - 2U * K), 768U);
+    else if constexpr (K == 4) go(tiled_step<T, Bounded, Forced, K, 34, 16>, kLargeRows, 1024U);
+    else throw std::invalid_argument("tiled_steps: two steps in one launch only on small lattices");
     if (const hipError_t e = hipGetLastError(); e != hipSuccess)
         throw std::runtime_error(std::string("tiled_step launch: ") + hipGetErrorString(e));
 }
@@ -213,10 +216,38 @@ template <class T> void steps(const LaunchState& st, int k, bool bounded, bool f
 
 }  // namespace
 
-bool tiled_supported(int q, int storage, size_t nx, size_t ny) {
-    // The coordinates wrap once, so the lattice is at least as large as the halo; FP64 stays with the
-    // single step (its tile would be half as large).
-    return q == 9 && (storage == 0 || storage == 1 || storage == 3) && nx >= 2 * kHalo && ny >= 2 * kHalo;
+// The coordinates wrap once, so the lattice is at least as large as the halo; FP64 stays with the single
+// step (its tile would be half as large).
+//
+// On small lattices both widths are ahead of the single step (64 000 cells of any shape: 4 steps 0.5-0.8 of
+// its time, 2 steps 0.6-0.95; only FP16S rows of 8 cells next to walls take 1.07 with 2).  In the large
+// tile 2 steps move nearly as much memory as 2 single ones and wait for it longer: 0.8-1.1 of the single
+// step's time in FP32, up to 1.5 in FP16S (4096^2 periodic 1.19, 128 x 62500 cavity 1.52), so what 4 steps
+// leave over runs singly there.
+//
+// 4 steps pay there by the wavefronts that a level issues for one of the single step (64-cell segments):
+// strips x (ny + 3 tile rows) / (segments x ny), 1.2 to 1.4 for most lattices, 1.67 for 128-wide rows, 2.2
+// for 57- to 64-wide ones.
+//  * FP32 and FP32S, unforced, are bound by memory as single steps: 0.4-0.8 of the single step's time, 0.6-0.97
+//    in 57- to 64-wide rows.  No limit.
+//  * Forced and LES steps issue more: 0.5-1.0 up to 1.67, 1.0-1.3 in 57- to 64-wide rows.  Limit 2.
+//  * FP16S moves half the bytes.  Periodic: 0.5-0.95 up to 1.67, 0.8-1.2 in 57- to 64-wide rows; limit 2.
+//    Next to walls: 0.6-0.95 up to 1.4, 0.8-1.19 in 128-wide rows, 1.0-1.46 in 57- to 64-wide ones; limit
+//    1.5, and 1.3 where one lattice fits the 256 MiB Infinity Cache but two do not, since only the single
+//    step is served from it (8 M cells, cavity: 100000 x 80 at 1.31 1.11, 256-wide at 1.39 1.02, 2048- and
+//    4096-wide at 1.29 0.86 and 0.82).
+bool tiled_pays(int q, int storage, size_t nx, size_t ny, size_t bytes, int k, bool bounded, bool forced) {
+    if (q != 9 || (storage != 0 && storage != 1 && storage != 3) || nx < 2 * kHalo || ny < 2 * kHalo) return false;
+    if (nx * ny < kLargeTileCells) return k == 2 || k == 4;
+    if (k != 4) return false;
+    const uint64_t strips = (nx + 55U) / 56U, segments = (nx + 63U) / 64U;
+    const uint64_t launched = strips * (ny + (kHalo - 1U) * ((ny + kLargeRows - 1U) / kLargeRows));
+    const uint64_t single = segments * ny;
+    if (storage == 1 && bounded) {
+        const uint64_t cache = uint64_t{256} << 20;
+        return 100U * launched < (bytes <= cache && 2U * bytes > cache ? 130U : 150U) * single;
+    }
+    return (!forced && storage != 1) || launched < 2U * single;
 }
 
 void tiled_steps(int storage, const LaunchState& st, int k, bool bounded, bool forced, const void* src, void* dst) {

@@ -5,8 +5,9 @@
 
 namespace cfd_hip {
 
-// Whether a lattice of `nx` x `ny` D2Q9 cells can be advanced by tiled_steps.
-bool tiled_supported(int q, int storage, size_t nx, size_t ny);
+// Whether tiled_steps can advance a lattice of `nx` x `ny` cells (population array of `bytes` bytes) by `k`
+// (2 or 4) steps a launch, faster than single steps.
+bool tiled_pays(int q, int storage, size_t nx, size_t ny, size_t bytes, int k, bool bounded, bool forced);
 
 // `k` steps (2 or 4) of a D2Q9 lattice from src (even parity) into dst, another array of the same
 // layout, asynchronously on st.stream.

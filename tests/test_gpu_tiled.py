@@ -114,3 +114,23 @@ def test_first_call_during_a_capture_of_another_stream(hip):
         one.step(1)
     for got, want in zip(_state(g), _state(one)):
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("shape,storage,scene,count,taken", [
+    ((60, 4000), "fp16s", "cavity", 8, False), ((60, 4000), "fp32", "cavity", 8, True),
+    ((60, 4000), "fp32", "forced", 8, False), ((64, 4000), "fp32", "les", 8, False),
+    ((65, 4000), "fp16s", "periodic", 8, True), ((60, 4000), "fp16s", "periodic", 8, False),
+    ((128, 2000), "fp16s", "cavity", 8, False), ((128, 2000), "fp16s", "periodic", 8, True),
+    ((128, 2000), "fp32", "forced", 8, True), ((449, 469), "fp32", "periodic", 7, False),
+    ((449, 469), "fp16s", "periodic", 8, True), ((100, 500), "fp16s", "periodic", 4, True),
+    ((100, 500), "fp16s", "periodic", 3, False), ((1000, 8000), "fp16s", "cavity", 8, True),
+    ((256, 31250), "fp16s", "cavity", 8, False), ((256, 31250), "fp16s", "periodic", 8, True)])
+def test_lattices_that_take_several_steps_a_launch(hip, shape, storage, scene, count, taken):
+    """The rule by width, storage, forcing and size: only lattices that gain take a second array."""
+    report("tiled_rule", shape=shape, storage=storage, scene=scene, count=count)
+    g = _solver(hip, shape, storage, scene)
+    before = g.resident_bytes()
+    g.step(count)
+    grown = g.resident_bytes() - before
+    assert grown >= g.population_bytes() if taken else grown == 0
+    g.close()
