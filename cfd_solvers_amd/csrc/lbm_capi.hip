@@ -8,6 +8,7 @@
 #include "../../include/cfd_lbm/c_api.h"
 #include "checkpoint_schedule.hpp"
 #include "device_memory.hpp"
+#include "launch_rules.hpp"
 #include "lbm_adjoint.hpp"
 #include "lbm_kernels.hpp"
 #include "lbm_tiled.hpp"
@@ -114,7 +115,12 @@ struct cfd_lbm_solver {
     size_t nx = 0, ny = 0, nz = 0, cells = 0;
     float tau = 0.6F, ax = 0, ay = 0, az = 0;
     size_t elem = 4, real = 4;
-    Geometry geo{}, step_geo{};
+    Geometry geo{};
+    struct StepTiles {  // of the step kernels, their occupancy cap and that of the transposed step
+        Geometry geo{};
+        uint32_t lds = 0, adjoint_lds = 0;
+    };
+    StepTiles step_tiles[2];  // periodic, bounded
     hipStream_t stream = nullptr;
     const KernelOps* ops = nullptr;
     DeviceBuffer<unsigned char> f, flags, links, link_vel, segments, solid_rho, gamma, lacc, macro, partial, reduce_out;
@@ -122,7 +128,6 @@ struct cfd_lbm_solver {
     float u_peak = 0.0F, rho_out = 1.0F;
     bool les = false;  // Smagorinsky LES (esoteric_pull.hpp:72-97, InPlaceLbmConfig::smagorinsky_les)
     uint64_t t = 0;
-    uint32_t step_lds = 0, step_lds_periodic = 0, adjoint_lds = 0;
     std::vector<uint8_t> host_flags;  // copy of the flags (empty: periodic)
     float last_forward_ms = 0.0F, last_reverse_ms = 0.0F;
     uint64_t last_forward_steps = 0;
@@ -204,10 +209,6 @@ struct cfd_lbm_solver {
             if (2U * geo.stride * elem > (uint64_t{1} << 32))
                 throw std::invalid_argument("lattice too large: two population planes must fit in 4 GiB");
         }
-        step_geo = geo;
-        const uint32_t width = step_width();
-        tile_geometry(step_geo, width, width < 256U ? 256U / width : 1U);
-        step_geo.xcd_group = xcd_group(true);
         // Resident wavefronts per SIMD of the step kernel, bounded and periodic, capped by reserving
         // LDS per block (160 KiB per CU; a 256-thread block puts one wave on each of the 4 SIMDs).
         // Measured on MI355X:
@@ -229,15 +230,6 @@ struct cfd_lbm_solver {
             waves_bounded = waves_periodic = 5;
         }
         if (const char* v = std::getenv("CFD_LBM_WAVES")) waves_bounded = waves_periodic = std::atol(v);
-        // A block of `threads` threads is threads / 256 wavefronts on each SIMD.
-        const long threads = static_cast<long>(step_geo.bx) * step_geo.by;
-        auto lds_cap = [threads](long w) {
-            if (w < 3 || w >= 8) return 0U;
-            const long blocks = std::max(1L, (w * 256 + threads / 2) / threads);
-            return static_cast<uint32_t>(std::min(163840 / blocks - 1024, 65536L));
-        };
-        step_lds = lds_cap(waves_bounded);
-        step_lds_periodic = lds_cap(waves_periodic);
         // The transposed step (adjoint) runs 6 (FP16) or 5 (FP32) waves per SIMD by its registers.
         // On HBM-bound lattices fewer measured faster: FP16 at 5 (768^3 sphere cluster: 20.6 ->
         // 19.6 ms; on 128^3, which the caches partly hold, slower: 76 -> 79 us), FP32 in plain planes
@@ -247,7 +239,16 @@ struct cfd_lbm_solver {
         if (storage == 1 && cells >= (size_t{1} << 24)) adjoint_waves = 5;
         else if (fp32_arith && !blocked) adjoint_waves = 3;
         if (const char* v = std::getenv("CFD_LBM_ADJOINT_WAVES")) adjoint_waves = std::atol(v);
-        adjoint_lds = lds_cap(adjoint_waves);
+        for (const bool b : {false, true}) {
+            StepTiles& s = step_tiles[b ? 1 : 0];
+            s.geo = geo;
+            const uint32_t width = step_width(b);
+            tile_geometry(s.geo, width, width < 256U ? 256U / width : 1U);
+            s.geo.xcd_group = xcd_group(s.geo.tiles, true);
+            const long threads = static_cast<long>(s.geo.bx) * s.geo.by;
+            s.lds = cfd_hip::occupancy_lds(b ? waves_bounded : waves_periodic, threads);
+            s.adjoint_lds = cfd_hip::occupancy_lds(adjoint_waves, threads);
+        }
 
         ops = cfd_hip::kernel_ops(q, storage);
         int count = 0;
@@ -285,32 +286,12 @@ struct cfd_lbm_solver {
         g.xcd_group = 0U;
     }
 
-    // Width of a step tile.  Neighbouring tiles of a row share cache lines at their common edge
-    // (populations are read and written at x - 1, x and x + 1), so a tile spans the row where a block
-    // can (256^3 cavity: 454 us a step with 256-wide tiles, 484 with 128, 563 with 64), and it launches
-    // no whole wavefronts beyond the row's end: five to eight 64-cell segments are one tile of just
-    // that width (301 x 150 x 141 FP32S: 190 us against 252 with 256-wide tiles, 203 with 128; 350 wide
-    // FP32: 216 against 287; 270 wide: 169 against 240).  Up to four segments take the 256-thread tile
-    // (192 wide, 192^3 FP32: 191 us with a 192-thread tile, 187 with 256).  Longer rows take the width
-    // that launches least, 256 unless that adds more than 1/8 to the row (2-D, 1100 wide: 25.4 us with
-    // 256, 26.1-27.4 with 320-512).  FP64 needs the registers of a 256-thread block, so its rows of
-    // more than four segments take 128 where that launches fewer (260 wide: 309 us against 405).
-    uint32_t step_width() const {
-        const uint32_t most = real == 8 ? 4U : 8U;  // kStepThreads / 64
+    uint32_t step_width(bool with_flags) const {
         if (const char* v = std::getenv("CFD_LBM_BX")) {  // tuning: 64, 128 or a multiple of 64 up to the most
-            const long w = std::atol(v);
-            if (w >= 64 && w <= 64 * static_cast<long>(most) && w % 64 == 0 && w != 192) return static_cast<uint32_t>(w);
+            const long w = std::atol(v), most = real == 8 ? 256 : 512;  // kStepThreads
+            if (w >= 64 && w <= most && w % 64 == 0 && w != 192) return static_cast<uint32_t>(w);
         }
-        const uint32_t segments_x = seg_x();
-        const auto launched = [segments_x](uint32_t w) { return (segments_x + w - 1U) / w * w; };
-        if (segments_x <= 4U) return geo.bx;
-        if (segments_x <= most) return 64U * segments_x;
-        if (real == 8) return launched(2U) < launched(4U) ? 128U : 256U;
-        if (launched(4U) * 8U <= segments_x * 9U) return 256U;
-        uint32_t best = 4U;
-        for (uint32_t w = 5U; w <= most; ++w)
-            if (launched(w) < launched(best)) best = w;
-        return 64U * best;
+        return cfd_hip::step_tile_width(seg_x(), elem, with_flags && geo.row_shift != 31);
     }
 
     // Consecutive tiles of one XCD in the step kernels.  A small lattice gives each XCD one run of rows:
@@ -330,13 +311,13 @@ struct cfd_lbm_solver {
     // lambda, so the caches hold none of them however small one is: in_place = false there (drag
     // gradient of 60 steps, 145^3 FP32: 25.3 ms in runs of 8, 27.0 in one run each; 96^3: 7.05
     // round-robin, 7.43).
-    uint32_t xcd_group(bool in_place) const {
-        const uint32_t run = (step_geo.tiles + 7U) / 8U;
+    uint32_t xcd_group(uint32_t tiles, bool in_place) const {
+        const uint32_t run = (tiles + 7U) / 8U;
         if (const char* v = std::getenv("CFD_LBM_XCD_REMAP")) {  // tuning: 0 round-robin, 1 one run each, n: n tiles
             const long g = std::atol(v);
             return g <= 0 ? 0U : (g == 1 ? run : static_cast<uint32_t>(std::min<long>(g, run)));
         }
-        if (step_geo.tiles > (1U << 22)) return 0U;  // the padding to whole runs stays far below the grid's limit
+        if (tiles > (1U << 22)) return 0U;  // the padding to whole runs stays far below the grid's limit
         const bool whole_lines = nx * elem % 128U == 0;
         const uint64_t bytes = pop_elems * elem;
         if (whole_lines && bytes <= (uint64_t{32} << 20)) return 0U;
@@ -383,8 +364,8 @@ struct cfd_lbm_solver {
     LaunchState state() {
         if (real == 8) build_physics<double>();
         else build_physics<float>();
-        return LaunchState{f.ptr, geo, step_geo, physics, stream, static_cast<uint32_t>(cells), step_lds, step_lds_periodic,
-                           adjoint_lds};
+        const StepTiles& s = step_tiles[bounded() ? 1 : 0];
+        return LaunchState{f.ptr, geo, s.geo, physics, stream, static_cast<uint32_t>(cells), s.lds, s.adjoint_lds};
     }
 
     void sync() const {
@@ -1019,7 +1000,7 @@ struct cfd_lbm_solver {
         args.grad_gamma = grad_on_device ? grad_gamma_out : reinterpret_cast<double*>(base + gg_at);
         args.grad_peak = reinterpret_cast<double*>(base + gp_at);
         LaunchState st = state();
-        st.step_geo.xcd_group = xcd_group(false);
+        st.step_geo.xcd_group = xcd_group(st.step_geo.tiles, false);
         adj->zero(st, args.grad_gamma, cells);
         adj->zero(st, args.grad_peak, cells);
         adj->zero(st, acc, 1);

@@ -652,8 +652,7 @@ template <int Q, class T> struct Ops final : KernelOps {
     template <bool Odd, bool Bounded, bool Forced>
     static void step_t(const LaunchState& st, const void* src, void* dst) {
         hipLaunchKernelGGL((stream_collide<Q, T, Odd, Bounded, Forced>), grid_of(st.step_geo),
-                           block_of(st.step_geo), Bounded ? st.step_lds : st.step_lds_periodic, st.stream, src, dst,
-                           st.step_geo,
+                           block_of(st.step_geo), st.step_lds, st.stream, src, dst, st.step_geo,
                            *static_cast<const Physics<Real>*>(st.physics));
     }
     void step(const LaunchState& st, bool odd, bool bounded, bool forced, const void* src, void* dst) const override {

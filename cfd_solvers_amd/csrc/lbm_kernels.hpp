@@ -17,8 +17,7 @@ struct LaunchState {
     const void* physics;     // Physics<float> or Physics<double> (host copy, passed by value)
     hipStream_t stream;
     uint32_t cells;
-    uint32_t step_lds;       // dynamic LDS bytes per bounded step-kernel block (occupancy cap; 0 = none)
-    uint32_t step_lds_periodic;  // the same for the periodic step
+    uint32_t step_lds;       // dynamic LDS bytes per step-kernel block (occupancy cap; 0 = none)
     uint32_t adjoint_lds;    // the same for the transposed step
 };
 
