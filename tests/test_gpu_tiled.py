@@ -134,3 +134,11 @@ def test_lattices_that_take_several_steps_a_launch(hip, shape, storage, scene, c
     grown = g.resident_bytes() - before
     assert grown >= g.population_bytes() if taken else grown == 0
     g.close()
+
+
+@pytest.mark.parametrize("storage", ["fp32", "fp16s"])
+@pytest.mark.parametrize("shape", [(57, 9), (448, 520)])
+def test_plain_planes(hip, monkeypatch, shape, storage):
+    """The layout of lattices beyond 4 GiB."""
+    monkeypatch.setenv("CFD_LBM_LAYOUT", "planes")
+    _compare(hip, shape, storage, "cavity", (8, 9))
