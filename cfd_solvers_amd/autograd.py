@@ -97,8 +97,9 @@ class LbmAdjointProblem:
         return s.objective_run(self.steps, self.window, self.objective, self.x_in, self._x_out())
 
     def run(self, gamma, u_peak: float):
-        """J, dJ/dgamma (float64, shape of gamma; a device tensor when gamma is one and the plan is
-        binomial, else a numpy array) and dJ/du_peak from one forward + adjoint run."""
+        """J, dJ/dgamma (float64, shape of gamma) and dJ/du_peak from one forward + adjoint run.  dJ/dgamma
+        is a numpy array, but a device tensor when gamma is one and the plan is binomial; ``lbm_objective``
+        keeps it on gamma's device under either plan."""
         J, grad, du = self._run(gamma, u_peak)
         if self.checkpoint_every > 0 and isinstance(grad, torch.Tensor):
             grad = grad.cpu().numpy()

@@ -130,7 +130,6 @@ __device__ __forceinline__ void store_cell(void* f, const Geometry& g, const Phy
                                            uint32_t n, uint32_t x, uint32_t y, uint32_t z,
                                            typename Storage<T>::Real rho, typename Storage<T>::Real (&fout)[Q],
                                            const PairSlots<Q>& s) {
-    using L = Lattice<Q>;
     using S = Storage<T>;
     if constexpr (Bounded) moving_wall_terms<Q, S>(p, s.desc, n, rho, fout);
     const uint32_t off_n = opaque_offset(s.self);

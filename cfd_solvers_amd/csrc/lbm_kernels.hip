@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void mark_segments(const uint8_t* __restrict__
 }
 
 // Sets kPorousSegment in the word of every row segment that holds a cell with gamma != 0 (after
-// mark_segments has written the spans).  Launched on the step's grid: each wavefront covers one
+// mark_segments has written the spans).  Launched on 256-thread tiles: each wavefront covers one
 // segment (bx >= 64), and its first lane, x = 64 * segment, owns the word.
 template <class Real>
 __global__ __launch_bounds__(256) void mark_porous_segments(const Real* __restrict__ gamma, const Geometry g,
