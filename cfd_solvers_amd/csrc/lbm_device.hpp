@@ -608,9 +608,9 @@ __device__ __forceinline__ void relax(Real (&f)[Q], Real rp, Real rho, Real ux, 
     } else {
         // equilibrium() of a pair at once: the opposite direction has cu' = -cu exactly, so that
         // 0.5 cu' cu' is 0.5 cu cu and 1 + cu' is 1 - cu, and every result is the single formula's.
-        // With the 2-D velocity's z quotient left out, 142 vector instructions a D2Q9 cell against 166:
-        // 40^3 464 us per 100 steps against 504, 64^3 724 against 740, 4096^2 cavity 20 steps 2.60 ms
-        // against 2.69.
+        // Vector instructions of the periodic step: D3Q19 397 against 430, D2Q9 205 against 219.  64^3 6.66
+        // us a step against 6.81, D3Q27 56^3 7.25 against 7.34, four D2Q9 steps a launch on a 4096^2 cavity
+        // 91.0 us a step against 95.8; larger lattices unchanged (256^3 cavity 453 us).
         f[0] = f[0] - omega * (f[0] - equilibrium<S, Q, 0>(rho, ux, uy, uz, uu));
         static_for<(Q - 1) / 2>([&](auto P) {
             constexpr int i = 2 * decltype(P)::value + 1;

@@ -159,15 +159,17 @@ __global__ __launch_bounds__(W* Rows) void tiled_step(const void* __restrict__ s
 constexpr uint32_t kHalo = 4;  // the largest K
 
 // Two tiles, both 64 slots (one wavefront) wide.  34 rows (FP32: 77 KiB of LDS, two blocks a CU)
-// recompute 18 % of the cells at K = 4 and are bound by the vector units: 4096^2 cavity FP32 134 us a
-// step against 201 single (periodic 127 against 201, FP16S 91 against 115), 1400^2 15.1 against 26.2.
-// 26 rows measure 137-142, 42 rows 152, 8 rows of threads instead of 16 139.
+// recompute 18 % of the cells at K = 4 and are bound by the vector units: 4096^2 cavity FP32 91 us a step
+// in calls of 40 against 196 single (periodic 83 against 204, FP16S 76 against 109), 1400^2 13.6 against
+// 24.0.  When they were chosen, at 134 us, 26 rows measured 137-142, 42 rows 152, 8 rows of threads
+// instead of 16 139.
 //
 // Below about 200 000 cells those tiles are too few to fill the chip, and the launch and the chain of
 // levels count: up to 16 rows, 12 of them at a time, and as many interior rows as make the fewest
-// wavefronts of the busiest CU (tile_rows).  256^2 FP32: 2.0 us a step against 4.2 single and 2.9 in
-// the large tile; 330^2: 2.2; 400^2: 2.6 against 5.5 and 3.0; 100 x 500: 1.9.  Tiles of 32 x 16 slots
-// measure 2.1, 2.4, 2.9 and 2.1; the large tile is ahead at 600^2 (3.6 against 4.6).
+// wavefronts of the busiest CU (tile_rows).  256^2 FP32 periodic: 1.8 us a step against 4.2 single; 330^2:
+// 2.0 against 3.9; 400^2: 2.1 against 3.9; 100 x 500: 1.7 against 4.1.  When they were chosen, at 2.0, 2.2,
+// 2.6 and 1.9, tiles of 32 x 16 slots measured 2.1, 2.4, 2.9 and 2.1, the large tile 2.9 at 256^2 and 3.0
+// at 400^2; it was ahead at 600^2 (3.6 against 4.6).
 constexpr uint32_t kLargeTileCells = 200000U;
 constexpr uint32_t kLargeRows = 34U - 2U * kHalo;  // interior rows of the large tile
 
