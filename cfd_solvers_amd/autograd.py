@@ -8,8 +8,9 @@ requires it), the same C-ABI call also runs the hand-written adjoint, so ``J.bac
 dJ/dgamma and dJ/du_peak without further GPU work; otherwise (``torch.no_grad()``, line searches,
 finite differences) only the steps and the objective run (``cfd_lbm_objective_run``), the same J
 bit for bit at the cost of the forward steps alone.  A ``gamma`` on the GPU stays there: the field
-is read from device memory and dJ/dgamma is written into a device tensor; no host round trip.  PyTorch is only the caller's interface here: the forward steps, the
-transposed steps and the checkpointing all run in ``libcfd_lbm_hip.so``.
+is read from device memory and dJ/dgamma is written into a device tensor; no host round trip.  PyTorch
+is only the caller's interface here: the forward steps, the transposed steps and the checkpointing all
+run in ``libcfd_lbm_hip.so``.
 
 The reference has no differentiable solver; the gradients are checked against central finite
 differences and the FP64 build of the same adjoint.
@@ -27,7 +28,17 @@ from typing import Optional
 import numpy as np
 import torch
 
-from .bindings import EsotericPullHipSolver, LATTICES
+from .bindings import EsotericPullHipSolver, LATTICES, release_workspaces
+
+
+def _with_room(allocate):
+    """``allocate()``, once more with the library's kept device memory given back if PyTorch's allocator
+    finds the device full: it cannot reclaim that memory itself."""
+    try:
+        return allocate()
+    except torch.cuda.OutOfMemoryError:
+        release_workspaces()
+        return allocate()
 
 
 @dataclass
@@ -76,7 +87,7 @@ class LbmAdjointProblem:
         s = self.solver()
         s.set_inlet_outlet(float(u_peak), self.rho_out)
         if isinstance(gamma, torch.Tensor) and gamma.is_cuda:
-            g = gamma.detach().to(torch.float32).contiguous().reshape(-1)
+            g = _with_room(lambda: gamma.detach().to(torch.float32).contiguous().reshape(-1))
             if g.numel() != s.cells:
                 raise ValueError("gamma must have one value per cell")
             torch.cuda.current_stream(g.device).synchronize()  # the library reads it on its own stream
@@ -112,7 +123,7 @@ class LbmAdjointProblem:
         if self.checkpoint_every > 0 and self.objective != "pressure_drop":
             raise ValueError("two-level checkpointing runs the pressure-drop objective; use checkpoint_every=0")
         if isinstance(gamma, torch.Tensor) and gamma.is_cuda:
-            grad = torch.empty(s.cells, dtype=torch.float64, device=gamma.device)
+            grad = _with_room(lambda: torch.empty(s.cells, dtype=torch.float64, device=gamma.device))
             torch.cuda.current_stream(grad.device).synchronize()  # its memory may still be in use there
             if self.checkpoint_every > 0:
                 J, du = s.adjoint_run_device(self.steps, self.window, self.checkpoint_every, grad.data_ptr(),
@@ -146,7 +157,7 @@ class LbmObjective(torch.autograd.Function):
         J, grad, du = problem._run(gamma, u)
         if not isinstance(grad, torch.Tensor):
             grad = torch.from_numpy(grad)
-        ctx.save_for_backward(grad.to(gamma.device, gamma.dtype),
+        ctx.save_for_backward(_with_room(lambda: grad.to(gamma.device, gamma.dtype)),
                               torch.tensor(du, dtype=u_peak.dtype, device=u_peak.device))
         return torch.tensor(J, dtype=torch.float64, device=gamma.device)
 
